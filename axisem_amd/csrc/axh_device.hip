@@ -95,9 +95,10 @@ constexpr uint8_t kFlagDirect = 64;   // one element copy and nothing else to ad
 constexpr int kMaxAxisBdry = 16;
 
 // kernel classes for timing
-// (the fluid stiffness is part of the stiffness launch; the solid-fluid
-// coupling and the symplectic drifts after the first are part of the
-// assemble_update kernels)
+// (the fluid stiffness and the coupling into the fluid are part of the
+// stiffness launch; the coupling into the solid and the symplectic drifts
+// after the first are part of the assembly launch, which is the solid's and
+// the fluid's together but for absorbing boundaries)
 enum KClass { KC_PRED = 0, KC_SOLID, KC_ASM_F, KC_ASM_S, KC_MEMVAR, KC_REC, KC_N };
 static const char *const kClassName[KC_N] = {
     "predict", "stiffness", "fluid_assemble_update", "solid_assemble_update",
@@ -161,7 +162,11 @@ struct MeshDev {
   int *einfo_f = nullptr, *gid_f = nullptr, *gstart_f = nullptr, *gslot_f = nullptr;
   uint8_t *flags_f = nullptr;
   // coupling
-  int *cpl_ss = nullptr, *cpl_gs = nullptr, *cpl_sf = nullptr, *cpl_gf = nullptr;
+  int *cpl_gs = nullptr, *cpl_gf = nullptr;
+  int *cpl_pt = nullptr;      // per solid point: the fluid point on it, or -1
+  // the fluid is assembled by a launch of its own before the solid: absorbing
+  // boundaries, or coupling entries of one solid point on several fluid points
+  bool split_asm = false;
   float *cpl_bm = nullptr;    // [nbdry*5][2]
   int *cpl_axb = nullptr;     // side-buffer slot of a masked axis point or -1
   int *axb_g = nullptr;       // global ids of the masked axis boundary points
@@ -312,6 +317,16 @@ struct FluidArgs {
   const float *stf[kGroup];  // NULL when the wavefield has no fluid source
   StepRef step;
   int nstages, stage;
+  // solid-fluid coupling (bdry_copy2fluid): added to the force of a coupled
+  // slot; the solid points it reads have several copies, so no lane of the
+  // launch writes their displacement
+  int dipole, nglob_s;
+  const int *cpl_slot;    // per fluid slot: coupling entry or -1 (NULL: none)
+  const int *cpl_gs;      // solid point of a coupling entry
+  const int *cpl_axb;     // its side-buffer slot or -1
+  const float *cpl_bm;    // [entry][2]
+  const float *disp;      // [3][nglob_s][B], the stage's prediction
+  const float *axb_val;   // [naxb][3][B]
 };
 
 // ---------------------------------------------------------------------------
@@ -587,8 +602,10 @@ __device__ __forceinline__ void gather_disp(const SolidArgs &A, bool valid, int 
 
 // ---------------------------------------------------------------------------
 // fluid stiffness glob_fluid_stiffness_4 (SOLVER/stiffness_fluid.f90:139-216)
-// + add_source_fl (SOLVER/time_evol_wave.F90:1062-1076) of one fluid tile; run
-// by the workgroups of the solid stiffness launch past the solid tiles
+// + add_source_fl (SOLVER/time_evol_wave.F90:1062-1076) + bdry_copy2fluid
+// (SOLVER/time_evol_wave.F90:1532-1580, with the prediction before the axis
+// mask) of one fluid tile; run by the workgroups of the solid stiffness launch
+// past the solid tiles
 // ---------------------------------------------------------------------------
 // LDS (the stiffness kernel's own arrays): sC 256*B, sS0/sS1 256*B each,
 // sG 105 floats, 16-byte aligned.
@@ -657,7 +674,30 @@ __device__ __forceinline__ void fluid_tile(const FluidArgs &A, int tile, float *
     }
     out[b] = loc;
   }
-  if (valid) stv<B>(A.force + slot * B, out);
+  if (!valid) return;
+  const int p = A.cpl_slot ? A.cpl_slot[slot] : -1;
+  if (p >= 0) {
+    const int gs = A.cpl_gs[p], kq = A.cpl_axb[p];
+    const float *u = A.disp + (size_t)gs * B;
+    size_t cs = (size_t)A.nglob_s * B;
+    if (kq >= 0) {
+      u = A.axb_val + (size_t)kq * 3 * B;
+      cs = B;
+    }
+    float s1[B], s2[B], s3[B];
+    ldv<B>(u, s1);
+    ldv<B>(u + cs, s2);
+    ldv<B>(u + 2 * cs, s3);
+    const float bm1 = A.cpl_bm[2 * p], bm2 = A.cpl_bm[2 * p + 1];
+#pragma unroll
+    for (int b = 0; b < B; b++) {
+      if (A.dipole)
+        out[b] = out[b] - bm1 * (s1[b] + s2[b]) - bm2 * s3[b];
+      else
+        out[b] = out[b] - bm1 * s1[b] - bm2 * s3[b];
+    }
+  }
+  stv<B>(A.force + slot * B, out);
 }
 
 // ---------------------------------------------------------------------------
@@ -1859,10 +1899,63 @@ struct AsmSolidArgs {
   // slot before the slot enters the sum
   int dipole;
   const int *cpl_slot;   // per solid slot: coupling entry or -1
-  const int *cpl_gf;     // fluid point of a coupling entry
   const float *cpl_bm;   // [entry][2]
+  // the potential's second derivative of this stage: read (written by an
+  // earlier launch) at the fluid point cpl_gf of each coupling entry, or NULL:
+  // formed here from the fluid forces of the one fluid point cpl_pt on a
+  // coupled solid point
   const float *ddchi;    // [nglob_f][B]
+  const int *cpl_gf, *cpl_pt;
 };
+
+struct AsmFluidArgs {
+  int n, newmark, mask_axis, mask_surface;
+  const int *gstart, *gslot;
+  const uint8_t *flags;
+  const float *minv;
+  const float *gamma;        // absorbing boundaries: damping factor per point, or NULL
+  double hdt, cv;
+  const float *force;        // [nslot_f][B], with the coupling terms
+  float *dchi, *ddchi;       // [n][B]
+  // symplectic: the drift of the next stage (or the final drift) right after
+  // the kick, chi = chi + dchi*cd_next, axis-masked when drift_mask is set
+  int drift, drift_mask;
+  double cd_next;
+  float *chi;                // [n][B]
+};
+
+// copies of a point gathered at a time
+template <int B>
+constexpr int kAsmChunk = (B >= 3 ? 2 : 4);
+
+// sum of the element forces of fluid point g (pdistsum_fluid), zero where
+// masked: kAsmChunk copies at a time (loads in flight together), summed in
+// ascending slot order from zero
+template <int B>
+__device__ __forceinline__ void fluid_sum(const AsmFluidArgs &A, int g, float (&s)[B]) {
+  const uint8_t fl = A.flags[g];
+  const bool masked = (A.mask_axis && (fl & kFlagAxis)) ||
+                      (A.mask_surface && (fl & kFlagSurface));
+#pragma unroll
+  for (int b = 0; b < B; b++) s[b] = 0.0f;
+  if (masked) return;
+  constexpr int W = kAsmChunk<B>;
+  const int q1 = A.gstart[g + 1];
+  for (int q = A.gstart[g]; q < q1; q += W) {
+    int sl[W];
+#pragma unroll
+    for (int w = 0; w < W; w++) sl[w] = (q + w < q1) ? A.gslot[q + w] : -1;
+    float x[W][B];
+#pragma unroll
+    for (int w = 0; w < W; w++)
+      if (sl[w] >= 0) ldv<B>(A.force + (size_t)sl[w] * B, x[w]);
+#pragma unroll
+    for (int w = 0; w < W; w++)
+      if (sl[w] >= 0)
+#pragma unroll
+        for (int b = 0; b < B; b++) s[b] = s[b] + x[w][b];
+  }
+}
 
 // The copies of a point are gathered kAsmChunk at a time with the three
 // components together, so that up to twelve loads are in flight per lane; each
@@ -1870,15 +1963,21 @@ struct AsmSolidArgs {
 // zero.  The point's velocity (and acceleration, displacement) is loaded
 // before the gather for the same reason.
 template <int B>
-constexpr int kAsmChunk = (B >= 3 ? 2 : 4);
-template <int B>
-__global__ __launch_bounds__(256) void k_asm_solid(AsmSolidArgs A) {
-  const int ip = xcd_block(blockIdx.x, gridDim.x) * 256 + threadIdx.x;
-  if (ip >= A.npts) return;
+__device__ __forceinline__ void asm_solid_point(const AsmSolidArgs &A, const AsmFluidArgs &FA,
+                                                int ip) {
   const int g = ip < A.ncontig ? ip : A.pts[ip];
   const uint8_t fl = A.flags[g];
   const int q0 = A.gstart[g], q1 = A.gstart[g + 1];
   const float mi = A.minv[g];
+  float f2[B];
+  if ((fl & kFlagCoupled) && !A.ddchi) {
+    // as the fluid lanes of this launch form it
+    const int gf = A.cpl_pt[g];
+    fluid_sum<B>(FA, gf, f2);
+    const float mf = FA.minv[gf];
+#pragma unroll
+    for (int b = 0; b < B; b++) f2[b] = -mf * f2[b];
+  }
   // a component is gathered unless it is off or axis-masked (masked copies
   // are zero before the gather)
   bool on[3];
@@ -1921,8 +2020,7 @@ __global__ __launch_bounds__(256) void k_asm_solid(AsmSolidArgs A) {
       for (int w = 0; w < W; w++) {
         const int p = sl[w] >= 0 ? A.cpl_slot[sl[w]] : -1;
         if (p < 0) continue;
-        float f2[B];
-        ldv<B>(A.ddchi + (size_t)A.cpl_gf[p] * B, f2);
+        if (A.ddchi) ldv<B>(A.ddchi + (size_t)A.cpl_gf[p] * B, f2);
         const float bm0 = A.cpl_bm[2 * p], bm1 = A.cpl_bm[2 * p + 1];
 #pragma unroll
         for (int c = 0; c < 3; c++) {
@@ -2003,89 +2101,10 @@ __global__ __launch_bounds__(256) void k_asm_solid(AsmSolidArgs A) {
   }
 }
 
-struct AsmFluidArgs {
-  int n, newmark, mask_axis, mask_surface;
-  const int *gstart, *gslot;
-  const uint8_t *flags;
-  const float *minv;
-  const float *gamma;        // absorbing boundaries: damping factor per point, or NULL
-  double hdt, cv;
-  const float *force;        // [nslot_f][B]
-  float *dchi, *ddchi;       // [n][B]
-  // symplectic: the drift of the next stage (or the final drift) right after
-  // the kick, chi = chi + dchi*cd_next, axis-masked when drift_mask is set
-  int drift, drift_mask;
-  double cd_next;
-  float *chi;                // [n][B]
-  // solid-fluid coupling (bdry_copy2fluid): added to the force of a coupled
-  // slot before the slot enters the sum
-  int dipole, nglob_s;
-  const int *cpl_slot;       // per fluid slot: coupling entry or -1
-  const int *cpl_gs;         // solid point of a coupling entry
-  const int *cpl_axb;        // its side-buffer slot or -1
-  const float *cpl_bm;       // [entry][2]
-  const float *disp;         // [3][nglob_s][B], the stage's prediction
-  const float *axb_val;      // [naxb][3][B]
-};
-
 template <int B>
-__global__ __launch_bounds__(256) void k_asm_fluid(AsmFluidArgs A) {
-  const int g = xcd_block(blockIdx.x, gridDim.x) * 256 + threadIdx.x;
-  if (g >= A.n) return;
-  const uint8_t fl = A.flags[g];
-  const bool masked = (A.mask_axis && (fl & kFlagAxis)) ||
-                      (A.mask_surface && (fl & kFlagSurface));
+__device__ __forceinline__ void asm_fluid_point(const AsmFluidArgs &A, int g) {
   float s[B];
-#pragma unroll
-  for (int b = 0; b < B; b++) s[b] = 0.0f;
-  if (!masked) {
-    // copies gathered four at a time (loads in flight together), summed in
-    // ascending slot order from zero
-    const bool coupled = fl & kFlagCoupled;
-    const int q1 = A.gstart[g + 1];
-    for (int q = A.gstart[g]; q < q1; q += 4) {
-      int sl[4];
-#pragma unroll
-      for (int w = 0; w < 4; w++) sl[w] = (q + w < q1) ? A.gslot[q + w] : -1;
-      float x[4][B];
-#pragma unroll
-      for (int w = 0; w < 4; w++)
-        if (sl[w] >= 0) ldv<B>(A.force + (size_t)sl[w] * B, x[w]);
-      if (coupled) {
-        // bdry_copy2fluid (SOLVER/time_evol_wave.F90:1532-1580) with the
-        // prediction before the axis mask
-#pragma unroll
-        for (int w = 0; w < 4; w++) {
-          const int p = sl[w] >= 0 ? A.cpl_slot[sl[w]] : -1;
-          if (p < 0) continue;
-          const int gs = A.cpl_gs[p], kq = A.cpl_axb[p];
-          float s1[B], s2[B], s3[B];
-          if (kq >= 0) {
-            ldv<B>(A.axb_val + ((size_t)kq * 3 + 0) * B, s1);
-            ldv<B>(A.axb_val + ((size_t)kq * 3 + 1) * B, s2);
-            ldv<B>(A.axb_val + ((size_t)kq * 3 + 2) * B, s3);
-          } else {
-            ldv<B>(A.disp + (size_t)gs * B, s1);
-            ldv<B>(A.disp + ((size_t)A.nglob_s + gs) * B, s2);
-            ldv<B>(A.disp + (2 * (size_t)A.nglob_s + gs) * B, s3);
-          }
-          const float bm1 = A.cpl_bm[2 * p], bm2 = A.cpl_bm[2 * p + 1];
-#pragma unroll
-          for (int b = 0; b < B; b++) {
-            if (A.dipole)
-              x[w][b] = x[w][b] - bm1 * (s1[b] + s2[b]) - bm2 * s3[b];
-            else
-              x[w][b] = x[w][b] - bm1 * s1[b] - bm2 * s3[b];
-          }
-        }
-      }
-#pragma unroll
-      for (int w = 0; w < 4; w++)
-        if (sl[w] >= 0)
-#pragma unroll
-          for (int b = 0; b < B; b++) s[b] = s[b] + x[w][b];
-    }
-  }
+  fluid_sum<B>(A, g, s);
   const float mi = A.minv[g];
   float d[B], dd[B], c[B];
   ldv<B>(A.dchi + (size_t)g * B, d);
@@ -2093,33 +2112,54 @@ __global__ __launch_bounds__(256) void k_asm_fluid(AsmFluidArgs A) {
   // absorbing boundaries: ddchi -= 2 gamma dchi + gamma^2 chi after the
   // inverse mass (SOLVER/time_evol_wave.F90:432-434,663-665)
   const float gm = A.gamma ? A.gamma[g] : 0.0f;
+#pragma unroll
+  for (int b = 0; b < B; b++) {
+    dd[b] = -mi * s[b];
+    if (A.gamma) dd[b] = (dd[b] - (2.0f * gm) * d[b]) - (gm * gm) * c[b];
+  }
   if (A.newmark) {
     float d0[B];
     ldv<B>(A.ddchi + (size_t)g * B, d0);
 #pragma unroll
-    for (int b = 0; b < B; b++) {
-      dd[b] = -mi * s[b];
-      if (A.gamma) dd[b] = (dd[b] - (2.0f * gm) * d[b]) - (gm * gm) * c[b];
+    for (int b = 0; b < B; b++)
       d[b] = (float)((double)d[b] + A.hdt * (double)(d0[b] + dd[b]));
-    }
   } else {
 #pragma unroll
-    for (int b = 0; b < B; b++) {
-      dd[b] = -s[b] * mi;
-      if (A.gamma) dd[b] = (dd[b] - (2.0f * gm) * d[b]) - (gm * gm) * c[b];
-      d[b] = (float)((double)d[b] + A.cv * (double)dd[b]);
-    }
+    for (int b = 0; b < B; b++) d[b] = (float)((double)d[b] + A.cv * (double)dd[b]);
   }
   stv<B>(A.ddchi + (size_t)g * B, dd);
   stv<B>(A.dchi + (size_t)g * B, d);
   if (A.drift) {
 #pragma unroll
     for (int b = 0; b < B; b++) c[b] = (float)((double)c[b] + (double)d[b] * A.cd_next);
-    if (A.drift_mask && (fl & kFlagAxis)) {
+    if (A.drift_mask && (A.flags[g] & kFlagAxis)) {
 #pragma unroll
       for (int b = 0; b < B; b++) c[b] = 0.0f;
     }
     stv<B>(A.chi + (size_t)g * B, c);
+  }
+}
+
+// The solid and the fluid assembly in one launch: nblk_s workgroups (a
+// multiple of the XCD count) take the solid points, the others the fluid
+// points.  They are independent: a coupled solid point forms the fluid's
+// second derivative it needs from the fluid forces itself (a few loads for
+// the points of the boundary, 0.1% of all), and the coupling into the fluid
+// is in the forces already.  The fluid assembly as a launch of its own before
+// the solid one costs 4.3 to 6.2 us per stage whatever the mesh size (launch
+// ramp and three dependent loads).  Two launches stay where that second
+// derivative depends on the fluid's state, which the fluid lanes overwrite
+// (absorbing boundaries), and where a solid point couples to several fluid
+// points (MeshDev::split_asm).
+template <int B>
+__global__ __launch_bounds__(256, (B >= 3 ? 5 : 6))
+void k_asm(AsmSolidArgs A, AsmFluidArgs F, int nblk_s) {
+  if ((int)blockIdx.x < nblk_s) {
+    const int ip = xcd_block(blockIdx.x, nblk_s) * 256 + threadIdx.x;
+    if (ip < A.npts) asm_solid_point<B>(A, F, ip);
+  } else {
+    const int g = xcd_block(blockIdx.x - nblk_s, gridDim.x - nblk_s) * 256 + threadIdx.x;
+    if (g < F.n) asm_fluid_point<B>(F, g);
   }
 }
 
@@ -2887,13 +2927,19 @@ static std::shared_ptr<MeshDev> mesh_build(const axh_ctx *ctx) {
     V.gslot_f = m.upload(H.gslot_f);
     V.minv_f = m.upload(H.minv_f);
     if (!H.gamma_f.empty()) V.gamma_f = m.upload(H.gamma_f);
+    V.split_asm = V.gamma_f != nullptr;
     V.flags_f = m.upload(H.flags_f);
   }
   if (V.nbdry > 0) {
-    V.cpl_ss = m.upload(H.cpl_ss);
     V.cpl_gs = m.upload(H.cpl_gs);
-    V.cpl_sf = m.upload(H.cpl_sf);
     V.cpl_gf = m.upload(H.cpl_gf);
+    std::vector<int> pt(V.nglob_s, -1);
+    for (size_t p = 0; p < H.cpl_gs.size(); p++) {
+      int &f = pt[H.cpl_gs[p]];
+      if (f >= 0 && f != H.cpl_gf[p]) V.split_asm = true;
+      f = H.cpl_gf[p];
+    }
+    V.cpl_pt = m.upload(pt);
     V.cpl_axb = m.upload(H.cpl_axb);
     V.cpl_bm = m.upload(H.cpl_bm);
     V.cpl_slot_s = m.upload(H.cpl_slot_s);
@@ -3667,17 +3713,19 @@ static void run_group(Runner &R, const MeshDev &M, Fields &F, Member *const *mb,
   AS.gamma = M.gamma_s;
   AS.force = F.force_s; AS.velo = F.velo; AS.acc0 = F.acc0;
   AS.disp = F.disp; AS.naxb = M.naxb; AS.axb_g = M.axb_g; AS.axb_val = F.axb_val;
-  AS.dipole = M.src == AXH_DIPOLE; AS.cpl_slot = M.cpl_slot_s; AS.cpl_gf = M.cpl_gf;
-  AS.cpl_bm = M.cpl_bm; AS.ddchi = F.ddchi;
+  AS.dipole = M.src == AXH_DIPOLE; AS.cpl_slot = M.cpl_slot_s; AS.cpl_pt = M.cpl_pt;
+  AS.cpl_bm = M.cpl_bm;
+  AS.cpl_gf = M.cpl_gf;
+  AS.ddchi = M.split_asm ? F.ddchi : nullptr;
   AsmFluidArgs AF{};
   AF.n = M.nglob_f; AF.newmark = newmark; AF.mask_axis = multipole;
   AF.mask_surface = newmark; AF.gstart = M.gstart_f; AF.gslot = M.gslot_f;
   AF.flags = M.flags_f; AF.minv = M.minv_f; AF.hdt = hdt; AF.force = F.force_f;
   AF.gamma = M.gamma_f;
   AF.dchi = F.dchi; AF.ddchi = F.ddchi; AF.chi = F.chi;
-  AF.dipole = M.src == AXH_DIPOLE; AF.nglob_s = M.nglob_s; AF.cpl_slot = M.cpl_slot_f;
-  AF.cpl_gs = M.cpl_gs; AF.cpl_axb = M.cpl_axb; AF.cpl_bm = M.cpl_bm; AF.disp = F.disp;
-  AF.axb_val = F.axb_val;
+  FA.dipole = M.src == AXH_DIPOLE; FA.nglob_s = M.nglob_s; FA.cpl_slot = M.cpl_slot_f;
+  FA.cpl_gs = M.cpl_gs; FA.cpl_axb = M.cpl_axb; FA.cpl_bm = M.cpl_bm; FA.disp = F.disp;
+  FA.axb_val = F.axb_val;
   RecArgs RA{};
   RA.src = M.src; RA.nglob = M.nglob_s; RA.disp = F.disp;
   int maxrec = 0;
@@ -3766,15 +3814,17 @@ static void run_group(Runner &R, const MeshDev &M, Fields &F, Member *const *mb,
           else dispatch_anel_full<true, false, B>(M, st_, AN);
         });
       }
-      if (M.nel_f > 0) {
-        AF.cv = newmark ? 0.0 : M.coefv[st];
+      AF.cv = AS.cv = newmark ? 0.0 : M.coefv[st];
+      const int nbs = (nblk(AS.npts) + kXcd - 1) / kXcd * kXcd;
+      const int nbf = M.nel_f > 0 ? nblk(AF.n) : 0;
+      if (M.split_asm) {
         L(KC_ASM_F, [&] {
-          hipLaunchKernelGGL(k_asm_fluid<B>, dim3(nblk(AF.n)), dim3(256), 0, st_, AF);
+          hipLaunchKernelGGL(k_asm<B>, dim3(nbf), dim3(256), 0, st_, AS, AF, 0);
         });
       }
-      AS.cv = newmark ? 0.0 : M.coefv[st];
       L(KC_ASM_S, [&] {
-        hipLaunchKernelGGL(k_asm_solid<B>, dim3(nblk(AS.npts)), dim3(256), 0, st_, AS);
+        hipLaunchKernelGGL(k_asm<B>, dim3(nbs + (M.split_asm ? 0 : nbf)), dim3(256), 0, st_, AS, AF,
+                           nbs);
       });
     }
     bool any = sample_all && maxrec > 0;
@@ -4352,7 +4402,8 @@ void footprint(axh_ctx *ctx, size_t *mesh_bytes, size_t *wave_bytes) {
   m += ns * nc * 4 + nel_s * 4 + nax * 50 * 4 + ns * 4 + (gs + 1) * 4 + nel_s * 25 * 4 + gs * 4;
   if (nel_f) m += nf * 4 * 4 + nel_f * 4 + nel_f * 5 * 4 + nf * 4 + (gf + 1) * 4 + nel_f * 25 * 4 +
                   gf * 4 + gf;
-  if (d.nel_bdry) m += (size_t)d.nel_bdry * 5 * (5 * 4 + 8) + kMaxAxisBdry * 4 + (ns + nf) * 4;
+  if (d.nel_bdry)
+    m += (size_t)d.nel_bdry * 5 * (3 * 4 + 8) + kMaxAxisBdry * 4 + (ns + nf + gs) * 4;
   if (d.anel) m += nel_s * (kCgStage + kCgUpd) * 16 + 2 * nel_s * d.n_sls * 8;
   size_t w = 3 * gs * 4 * 3 + 3 * ns * 4 + 3 * kMaxAxisBdry * 4 + gs + gs * 4;
   if (nel_f) w += 3 * gf * 4 + nf * 4 + nel_f * 4 + 200 * 4;
