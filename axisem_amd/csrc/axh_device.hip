@@ -304,6 +304,13 @@ struct SolidArgs {
   float *velo, *acc0;     // [3][nglob][B]
   float *disp_w;          // disp, written by the drift
   double hdt, cv, cd_next;
+  // the next step's predictor (first drift) of the direct points, into the
+  // other displacement buffer; NULL: none
+  float *disp_next;
+  double dt, hdt2, cd0;
+  int *blow;
+  double thr;
+  StepRef step;
 };
 
 struct FluidArgs {
@@ -1257,6 +1264,14 @@ void k_solid(SolidArgs A, FluidArgs FA) {
           }
           stv<B>(A.acc0 + p, a);
           stv<B>(A.velo + p, dv[cc]);
+          if (A.disp_next) {
+            // k_predict of the next step (point (1,1) is lane k = 6)
+            const float u = sU[cc * 256 * B + t * B];
+            if (k == 6 && (double)fabsf(u) > A.thr)
+              atomicMin(A.blow, step_of(A.step, 0) + 1);
+            const float un = (float)((double)u + A.dt * (double)v[0] + A.hdt2 * (double)a[0]);
+            A.disp_next[p] = un;
+          }
         } else {
           float u[B];
 #pragma unroll
@@ -1270,6 +1285,11 @@ void k_solid(SolidArgs A, FluidArgs FA) {
           }
           stv<B>(A.velo + p, dv[cc]);
           stv<B>(A.disp_w + p, u);
+          if (A.disp_next) {
+            if (k == 6 && (double)fabsf(u[0]) > A.thr)
+              atomicMin(A.blow, step_of(A.step, 0) + 1);
+            A.disp_next[p] = (float)((double)u[0] + (double)v[0] * A.cd0);
+          }
         }
       }
     } else {
@@ -1810,7 +1830,8 @@ struct PredArgs {
   double dt, hdt2, cd;
   const uint8_t *flags;
   const int *axb_g;      // masked axis points on the solid-fluid boundary
-  float *u, *v;          // [comp][stride][B]
+  const float *u, *v;    // [comp][stride][B]
+  float *u_out;          // the prediction (u itself or the other buffer)
   const float *a0;
   float *axb_val;        // unmasked prediction of the axb points [naxb][3][B]
   int *blow[kGroup];
@@ -1850,7 +1871,7 @@ __device__ __forceinline__ void predict_point(const PredArgs &A, int g) {
 #pragma unroll
       for (int b = 0; b < B; b++) un[b] = 0.0f;
     }
-    stv<B>(A.u + p, un);
+    stv<B>(A.u_out + p, un);
   }
 }
 
@@ -1893,6 +1914,12 @@ struct AsmSolidArgs {
   int drift, drift_mask, naxb;
   double cd_next;
   float *disp;           // [3][n][B]
+  // the next step's predictor (first drift) with the axis mask and the
+  // blow-up test, into the other displacement buffer; NULL: none
+  float *disp_next;
+  double dt, hdt2, cd0;
+  int *blow[kGroup];
+  double thr[kGroup];
   const int *axb_g;
   float *axb_val;        // [naxb][3][B]
   // solid-fluid coupling (bdry_copy2solid): added to the force of a coupled
@@ -1922,6 +1949,10 @@ struct AsmFluidArgs {
   int drift, drift_mask;
   double cd_next;
   float *chi;                // [n][B]
+  // the next step's predictor (first drift), axis-masked with mask_axis, into
+  // the other buffer; NULL: none
+  float *chi_next;
+  double dt, hdt2, cd0;
 };
 
 // copies of a point gathered at a time
@@ -1991,7 +2022,7 @@ __device__ __forceinline__ void asm_solid_point(const AsmSolidArgs &A, const Asm
     const size_t p = ((size_t)c * A.n + g) * B;
     ldv<B>(A.velo + p, v[c]);
     if (A.newmark) ldv<B>(A.acc0 + p, a0[c]);
-    if (A.drift || A.gamma) ldv<B>(A.disp + p, u[c]);
+    if (A.drift || A.gamma || A.disp_next) ldv<B>(A.disp + p, u[c]);
   }
   // absorbing boundaries: a -= 2 gamma v + gamma^2 u after the inverse mass
   // (SOLVER/time_evol_wave.F90:468-491,690-711), with v and u of this stage
@@ -2059,8 +2090,8 @@ __device__ __forceinline__ void asm_solid_point(const AsmSolidArgs &A, const Asm
     for (int b = 0; b < B; b++)
       if (si[b] >= 0) s[c][b] = s[c][b] - A.src_val[b][3 * si[b] + c] * stf[b];
     const size_t p = ((size_t)c * A.n + g) * B;
+    float a[B];
     if (A.newmark) {
-      float a[B];
 #pragma unroll
       for (int b = 0; b < B; b++) {
         if (c == 2 && A.src == AXH_DIPOLE)
@@ -2074,12 +2105,12 @@ __device__ __forceinline__ void asm_solid_point(const AsmSolidArgs &A, const Asm
     } else {
 #pragma unroll
       for (int b = 0; b < B; b++) {
-        float a = -mi * s[c][b];
-        if (A.gamma) a = (a - (2.0f * gm) * v[c][b]) - (gm * gm) * u[c][b];
+        a[b] = -mi * s[c][b];
+        if (A.gamma) a[b] = (a[b] - (2.0f * gm) * v[c][b]) - (gm * gm) * u[c][b];
         if (c == 2 && A.src == AXH_DIPOLE)
-          v[c][b] = (float)((double)v[c][b] + 2.0 * (double)a * A.cv);
+          v[c][b] = (float)((double)v[c][b] + 2.0 * (double)a[b] * A.cv);
         else
-          v[c][b] = (float)((double)v[c][b] + (double)a * A.cv);
+          v[c][b] = (float)((double)v[c][b] + (double)a[b] * A.cv);
       }
     }
     stv<B>(A.velo + p, v[c]);
@@ -2098,6 +2129,28 @@ __device__ __forceinline__ void asm_solid_point(const AsmSolidArgs &A, const Asm
       }
       stv<B>(A.disp + p, u[c]);
     }
+    if (A.disp_next) {
+      // as k_predict, with the state just computed
+      if (fl & kFlagBlow) {
+#pragma unroll
+        for (int b = 0; b < B; b++)
+          if ((double)fabsf(u[c][b]) > A.thr[b]) atomicMin(A.blow[b], step_of(A.step, b) + 1);
+      }
+#pragma unroll
+      for (int b = 0; b < B; b++)
+        u[c][b] = A.newmark ? (float)((double)u[c][b] + A.dt * (double)v[c][b] +
+                                      A.hdt2 * (double)a[b])
+                            : (float)((double)u[c][b] + (double)v[c][b] * A.cd0);
+      if (fl & kFlagAxisBdry) {
+        for (int k = 0; k < A.naxb; k++)
+          if (A.axb_g[k] == g) stv<B>(A.axb_val + ((size_t)k * 3 + c) * B, u[c]);
+      }
+      if ((fl & kFlagAxis) && c >= A.mask0 && c <= A.mask1) {
+#pragma unroll
+        for (int b = 0; b < B; b++) u[c][b] = 0.0f;
+      }
+      stv<B>(A.disp_next + p, u[c]);
+    }
   }
 }
 
@@ -2108,7 +2161,7 @@ __device__ __forceinline__ void asm_fluid_point(const AsmFluidArgs &A, int g) {
   const float mi = A.minv[g];
   float d[B], dd[B], c[B];
   ldv<B>(A.dchi + (size_t)g * B, d);
-  if (A.drift || A.gamma) ldv<B>(A.chi + (size_t)g * B, c);
+  if (A.drift || A.gamma || A.chi_next) ldv<B>(A.chi + (size_t)g * B, c);
   // absorbing boundaries: ddchi -= 2 gamma dchi + gamma^2 chi after the
   // inverse mass (SOLVER/time_evol_wave.F90:432-434,663-665)
   const float gm = A.gamma ? A.gamma[g] : 0.0f;
@@ -2138,28 +2191,15 @@ __device__ __forceinline__ void asm_fluid_point(const AsmFluidArgs &A, int g) {
     }
     stv<B>(A.chi + (size_t)g * B, c);
   }
-}
-
-// The solid and the fluid assembly in one launch: nblk_s workgroups (a
-// multiple of the XCD count) take the solid points, the others the fluid
-// points.  They are independent: a coupled solid point forms the fluid's
-// second derivative it needs from the fluid forces itself (a few loads for
-// the points of the boundary, 0.1% of all), and the coupling into the fluid
-// is in the forces already.  The fluid assembly as a launch of its own before
-// the solid one costs 4.3 to 6.2 us per stage whatever the mesh size (launch
-// ramp and three dependent loads).  Two launches stay where that second
-// derivative depends on the fluid's state, which the fluid lanes overwrite
-// (absorbing boundaries), and where a solid point couples to several fluid
-// points (MeshDev::split_asm).
-template <int B>
-__global__ __launch_bounds__(256, (B >= 3 ? 5 : 6))
-void k_asm(AsmSolidArgs A, AsmFluidArgs F, int nblk_s) {
-  if ((int)blockIdx.x < nblk_s) {
-    const int ip = xcd_block(blockIdx.x, nblk_s) * 256 + threadIdx.x;
-    if (ip < A.npts) asm_solid_point<B>(A, F, ip);
-  } else {
-    const int g = xcd_block(blockIdx.x - nblk_s, gridDim.x - nblk_s) * 256 + threadIdx.x;
-    if (g < F.n) asm_fluid_point<B>(F, g);
+  if (A.chi_next) {
+    const bool masked = A.mask_axis && (A.flags[g] & kFlagAxis);
+#pragma unroll
+    for (int b = 0; b < B; b++) {
+      c[b] = A.newmark ? (float)((double)c[b] + A.dt * (double)d[b] + A.hdt2 * (double)dd[b])
+                       : (float)((double)c[b] + (double)d[b] * A.cd0);
+      if (masked) c[b] = 0.0f;
+    }
+    stv<B>(A.chi_next + (size_t)g * B, c);
   }
 }
 
@@ -2199,16 +2239,16 @@ struct KwfArgs {
   StepRef step;
 };
 
+// (workgroup blk of nblk)
 template <int B>
-__global__ __launch_bounds__(256) void k_kwf(KwfArgs A) {
-  const int b = blockIdx.y;
+__device__ __forceinline__ void kwf_points(const KwfArgs &A, int b, int blk, int nblk) {
   const int iter = step_of(A.step, b);
   // uniform per block: not a snapshot step of this wavefield
   if (iter % A.strain_it != 0 || (A.init_only && iter != 0)) return;
   float *o = A.ring[b] + (size_t)((iter / A.strain_it) % A.cap) * A.ncomp * A.npt;
   const int npf = A.npt - A.nps;
   const int *sol_g = A.sol_g[b];
-  for (int k = blockIdx.x * 256 + threadIdx.x; k < A.npt; k += gridDim.x * 256) {
+  for (int k = blk * 256 + threadIdx.x; k < A.npt; k += nblk * 256) {
     float s, p, z;
     if (k < A.nps) {
       const int g = sol_g[k];
@@ -2251,6 +2291,58 @@ __global__ __launch_bounds__(256) void k_kwf(KwfArgs A) {
       o[(size_t)A.npt + k] = z;
     }
   }
+}
+
+template <int B>
+__global__ __launch_bounds__(256) void k_kwf(KwfArgs A) {
+  kwf_points<B>(A, blockIdx.y, blockIdx.x, gridDim.x);
+}
+
+// The solid and the fluid assembly in one launch: nblk_s workgroups (a
+// multiple of the XCD count) take the solid points, the others the fluid
+// points.  They are independent: a coupled solid point forms the fluid's
+// second derivative it needs from the fluid forces itself (a few loads for
+// the points of the boundary, 0.1% of all), and the coupling into the fluid
+// is in the forces already.  The fluid assembly as a launch of its own before
+// the solid one costs 4.3 to 6.2 us per stage whatever the mesh size (launch
+// ramp and three dependent loads).  Two launches stay where that second
+// derivative depends on the fluid's state, which the fluid lanes overwrite
+// (absorbing boundaries), and where a solid point couples to several fluid
+// points (MeshDev::split_asm).
+//
+// The launch also forms the next step's prediction (disp_next, chi_next), so
+// that only the first step of a run or graph launches k_predict, and, for
+// newmark2, whose displacement of the step it does not write, takes the
+// step's receiver samples (nrec workgroups per wavefield) and kernel
+// wavefields (nkwf per wavefield).
+// workgroups of k_asm: solid points, fluid points, receivers and kernel
+// wavefields (the last two per wavefield)
+struct AsmBlocks {
+  int solid, fluid, rec, kwf;
+};
+
+template <int B>
+__global__ __launch_bounds__(256, (B >= 3 ? 5 : 6))
+void k_asm(AsmSolidArgs A, AsmFluidArgs F, RecArgs R, KwfArgs K, AsmBlocks N) {
+  int blk = blockIdx.x;
+  if (blk < N.solid) {
+    const int ip = xcd_block(blk, N.solid) * 256 + threadIdx.x;
+    if (ip < A.npts) asm_solid_point<B>(A, F, ip);
+    return;
+  }
+  blk -= N.solid;
+  if (blk < N.fluid) {
+    const int g = xcd_block(blk, N.fluid) * 256 + threadIdx.x;
+    if (g < F.n) asm_fluid_point<B>(F, g);
+    return;
+  }
+  blk -= N.fluid;
+  if (blk < N.rec * B) {
+    rec_sample<B>(R, (blk / B) * 256 + threadIdx.x, blk % B);
+    return;
+  }
+  blk -= N.rec * B;
+  kwf_points<B>(K, blk % B, blk / B, N.kwf);
 }
 
 // Start of a run: each wavefield's first step and its blow-up flag cleared
@@ -3000,6 +3092,10 @@ struct Fields {
   DevAlloc mem;
   float *disp = nullptr, *velo = nullptr, *acc0 = nullptr, *force_s = nullptr;
   float *chi = nullptr, *dchi = nullptr, *ddchi = nullptr, *force_f = nullptr;
+  // second buffers of disp and chi: within a run the steps alternate between
+  // the two (each step's launches write the next step's prediction into the
+  // other); every run starts and ends in disp, chi
+  float *disp2 = nullptr, *chi2 = nullptr;
   float *memvar = nullptr, *rsum = nullptr, *trm1 = nullptr, *devm1 = nullptr;
   float *axb_val = nullptr;   // unmasked prediction of the axis boundary points
   // solid point flags with the source points of the group's wavefields
@@ -3090,12 +3186,14 @@ static void fields_alloc(const MeshDev &M, Fields &F, int B) {
   F.step_base = m.zeros<int>(kGroup);
   const size_t b = B;
   F.disp = m.zeros<float>(3 * (size_t)M.nglob_s * b);
+  F.disp2 = m.zeros<float>(3 * (size_t)M.nglob_s * b);
   F.velo = m.zeros<float>(3 * (size_t)M.nglob_s * b);
   F.acc0 = m.zeros<float>(3 * (size_t)M.nglob_s * b);
   F.force_s = m.zeros<float>(3 * (size_t)M.ntile_s * kTile * b);
   F.axb_val = m.zeros<float>(3 * (size_t)std::max(M.naxb, 1) * b);
   if (M.nel_f > 0) {
     F.chi = m.zeros<float>((size_t)M.nglob_f * b);
+    F.chi2 = m.zeros<float>((size_t)M.nglob_f * b);
     F.dchi = m.zeros<float>((size_t)M.nglob_f * b);
     F.ddchi = m.zeros<float>((size_t)M.nglob_f * b);
     F.force_f = m.zeros<float>((size_t)M.ntile_f * kTile * b);
@@ -3665,7 +3763,7 @@ static void run_group(Runner &R, const MeshDev &M, Fields &F, Member *const *mb,
   for (int s = 0; s < kMaxSls; s++) {
     SA.expw[s] = M.expw[s]; SA.tst[s] = M.tst[s]; SA.tstm1[s] = M.tstm1[s];
   }
-  SA.disp = F.disp; SA.force = F.force_s; SA.memvar = F.memvar; SA.rsum = F.rsum;
+  SA.force = F.force_s; SA.memvar = F.memvar; SA.rsum = F.rsum;
   SA.trm1 = F.trm1; SA.devm1 = F.devm1;
   SA.flags = F.flags_s; SA.minv = M.minv_s; SA.velo = F.velo; SA.acc0 = F.acc0;
   SA.first_direct = M.first_direct;
@@ -3673,7 +3771,8 @@ static void run_group(Runner &R, const MeshDev &M, Fields &F, Member *const *mb,
     fail(AXH_ERR_STATE, "source points in more tiles than the group's source elements");
   SA.nsrc_tile = (int)F.src_tiles.size();
   for (size_t q = 0; q < F.src_tiles.size(); q++) SA.src_tile[q] = F.src_tiles[q];
-  SA.disp_w = F.disp; SA.hdt = hdt;
+  SA.hdt = hdt; SA.dt = dt; SA.hdt2 = hdt2; SA.cd0 = newmark ? 0.0 : M.coefd[0];
+  SA.blow = RB.blow[0]; SA.thr = mb[0]->blow_thr;
   AnelFullArgs AN{};
   if (M.anel_full) {
     AN.nel = M.nel_s; AN.nsls = M.nsls; AN.nglob = M.nglob_s; AN.nslot = (int)nslot_s;
@@ -3682,12 +3781,12 @@ static void run_group(Runner &R, const MeshDev &M, Fields &F, Member *const *mb,
     for (int s = 0; s < kMaxSls; s++) {
       AN.expw[s] = M.expw[s]; AN.tst[s] = M.tst[s]; AN.tstm1[s] = M.tstm1[s];
     }
-    AN.disp = F.disp; AN.force = F.force_s; AN.memvar = F.memvar; AN.trm1 = F.trm1;
+    AN.force = F.force_s; AN.memvar = F.memvar; AN.trm1 = F.trm1;
     AN.devm1 = F.devm1; AN.rsum = F.rsum;
   }
   FluidArgs FA{};
   FA.nel = M.nel_f; FA.multipole = multipole; FA.G = M.G; FA.coef = M.coef_f;
-  FA.m0 = M.m0_f; FA.einfo = M.einfo_f; FA.gid = M.gid_f; FA.chi = F.chi;
+  FA.m0 = M.m0_f; FA.einfo = M.einfo_f; FA.gid = M.gid_f;
   FA.force = F.force_f;
   // solid axis masks: monopole s; dipole +,z (2,3); quadrupole all
   const int mask0 = (M.src == AXH_DIPOLE) ? 1 : 0;
@@ -3712,7 +3811,7 @@ static void run_group(Runner &R, const MeshDev &M, Fields &F, Member *const *mb,
   AS.gslot = M.gslot_s; AS.flags = F.flags_s; AS.minv = M.minv_s; AS.hdt = hdt;
   AS.gamma = M.gamma_s;
   AS.force = F.force_s; AS.velo = F.velo; AS.acc0 = F.acc0;
-  AS.disp = F.disp; AS.naxb = M.naxb; AS.axb_g = M.axb_g; AS.axb_val = F.axb_val;
+  AS.dt = dt; AS.hdt2 = hdt2; AS.cd0 = SA.cd0; AS.naxb = M.naxb; AS.axb_g = M.axb_g; AS.axb_val = F.axb_val;
   AS.dipole = M.src == AXH_DIPOLE; AS.cpl_slot = M.cpl_slot_s; AS.cpl_pt = M.cpl_pt;
   AS.cpl_bm = M.cpl_bm;
   AS.cpl_gf = M.cpl_gf;
@@ -3722,18 +3821,19 @@ static void run_group(Runner &R, const MeshDev &M, Fields &F, Member *const *mb,
   AF.mask_surface = newmark; AF.gstart = M.gstart_f; AF.gslot = M.gslot_f;
   AF.flags = M.flags_f; AF.minv = M.minv_f; AF.hdt = hdt; AF.force = F.force_f;
   AF.gamma = M.gamma_f;
-  AF.dchi = F.dchi; AF.ddchi = F.ddchi; AF.chi = F.chi;
+  AF.dchi = F.dchi; AF.ddchi = F.ddchi; AF.dt = dt; AF.hdt2 = hdt2; AF.cd0 = SA.cd0;
   FA.dipole = M.src == AXH_DIPOLE; FA.nglob_s = M.nglob_s; FA.cpl_slot = M.cpl_slot_f;
-  FA.cpl_gs = M.cpl_gs; FA.cpl_axb = M.cpl_axb; FA.cpl_bm = M.cpl_bm; FA.disp = F.disp;
+  FA.cpl_gs = M.cpl_gs; FA.cpl_axb = M.cpl_axb; FA.cpl_bm = M.cpl_bm;
   FA.axb_val = F.axb_val;
   RecArgs RA{};
-  RA.src = M.src; RA.nglob = M.nglob_s; RA.disp = F.disp;
+  RA.src = M.src; RA.nglob = M.nglob_s;
   int maxrec = 0;
   for (int b = 0; b < B; b++) {
     Member &w = *mb[b];
     FA.srcel[b] = w.srcel_f; FA.src_fl[b] = w.src_fl;
     PS.blow[b] = RB.blow[b]; PS.thr[b] = w.blow_thr;
     PF.blow[b] = RB.blow[b]; PF.thr[b] = w.blow_thr;
+    AS.blow[b] = RB.blow[b]; AS.thr[b] = w.blow_thr;
     AS.nsrc[b] = w.nsrc; AS.src_g[b] = w.src_g; AS.src_val[b] = w.src_val;
     RA.nrec[b] = w.nrec; RA.rec_g[b] = w.rec_g; RA.ring[b] = RB.ring[b];
     RA.seis_it[b] = std::max(w.seis_it, 1); RA.cap[b] = RB.cap[b];
@@ -3750,7 +3850,7 @@ static void run_group(Runner &R, const MeshDev &M, Fields &F, Member *const *mb,
     T.q0[b] = T.qdone[b] = T.qout[b] = (start[b] - 1) / si;
   }
   const StepRef sref{RB.step_base, 0};
-  PS.step = PF.step = FA.step = AS.step = RA.step = sref;
+  PS.step = PF.step = FA.step = AS.step = RA.step = SA.step = sref;
   KwfArgs KA{};
   const int kwf_blocks = kw ? std::max(1, std::min(kKwfBlocks, nblk(kw->args.npt))) : 0;
   if (kw) {
@@ -3774,34 +3874,57 @@ static void run_group(Runner &R, const MeshDev &M, Fields &F, Member *const *mb,
     FA.stf[b] = (newmark && mb[b]->fluid_src) ? mb[b]->stf_d : nullptr;
     AS.stf[b] = (newmark && mb[b]->fluid_src) ? nullptr : mb[b]->stf_d;
   }
-  // the launches of the step koff steps past the step base; with sample_all
-  // the receiver kernels run every step (a graph's steps are all alike), else
-  // only where a wavefield takes a sample (it: the step on the host)
-  auto one_step = [&](int koff, bool sample_all, int step) {
-    PS.step.koff = PF.step.koff = FA.step.koff = AS.step.koff = RA.step.koff = koff;
+  // the launches of step k of a segment of n steps (koff = k steps past the
+  // step base).  The first step starts with k_predict; every other step but
+  // the last finds its prediction written by the step before, in the other
+  // buffer of disp and chi.  k_predict writes the buffer from which the
+  // segment's last step ends in disp, chi.  With sample_all the receiver
+  // samples are taken every step (a graph's steps are all alike), else only
+  // where a wavefield takes one (step: the run's step on the host)
+  float *const dbuf[2] = {F.disp, F.disp2}, *const cbuf[2] = {F.chi, F.chi2};
+  auto one_step = [&](int k, int n, bool sample_all, int step) {
+    PS.step.koff = PF.step.koff = FA.step.koff = AS.step.koff = RA.step.koff = k;
+    SA.step.koff = KA.step.koff = k;
+    const int cur = (n - 1 - k) & 1;
+    const bool ahead = k + 1 < n;   // the next step's prediction is formed here
+    float *const u = dbuf[cur], *const c = cbuf[cur];
+    SA.disp = SA.disp_w = AS.disp = u;
+    FA.disp = RA.disp = AN.disp = KA.disp = u;
+    FA.chi = AF.chi = c;
+    KA.chi = c;
+    if (k == 0) {
+      PS.newmark = PF.newmark = newmark;
+      PS.cd = PF.cd = newmark ? 0.0 : M.coefd[0];
+      PS.apply_mask = 1;
+      PF.apply_mask = multipole;
+      PS.check_blow = 1;
+      PF.check_blow = 0;
+      PS.u_out = u;
+      PF.u_out = c;
+      L(KC_PRED, [&] {
+        const int nbs = nblk(PS.n), nbf = M.nel_f > 0 ? nblk(PF.n) : 0;
+        hipLaunchKernelGGL(k_predict<B>, dim3(nbs + nbf), dim3(256), 0, st_, PS, PF, nbs);
+      });
+    }
+    bool any = sample_all && maxrec > 0;
+    for (int b = 0; b < B && !any; b++)
+      any = mb[b]->nrec > 0 && (start[b] + step) % mb[b]->seis_it == 0;
+    // kernel-wavefield snapshot of the step (a graph's steps all launch it;
+    // its workgroups return at once where the step is not a snapshot step)
+    bool snap = kw && KA.npt > 0 && sample_all;
+    for (int b = 0; b < B && kw && KA.npt > 0 && !snap; b++)
+      snap = (start[b] + step) % KA.strain_it == 0;
     for (int st = 0; st < M.nstages; st++) {
-      // predictor / first drift of the step; the symplectic drifts of the
-      // later stages and the final drift are fused into the kicks below
-      if (newmark || st == 0) {
-        PS.newmark = PF.newmark = newmark;
-        PS.cd = PF.cd = newmark ? 0.0 : M.coefd[st];
-        PS.apply_mask = 1;
-        PF.apply_mask = multipole;
-        PS.check_blow = 1;
-        PF.check_blow = 0;
-        L(KC_PRED, [&] {
-          const int nbs = nblk(PS.n), nbf = M.nel_f > 0 ? nblk(PF.n) : 0;
-          hipLaunchKernelGGL(k_predict<B>, dim3(nbs + nbf), dim3(256), 0, st_, PS, PF, nbs);
-        });
-      }
-      // drift after the kick: coefd(st+1), masked except the final one
-      // (SOLVER/time_evol_wave.F90:597-605,720-725)
+      // the drifts after the first are fused into the kicks: coefd(st+1),
+      // masked except the final one (SOLVER/time_evol_wave.F90:597-605,720-725)
       const bool last = st + 1 == M.nstages;
       AS.drift = AF.drift = !newmark;
       AS.cd_next = AF.cd_next = newmark ? 0.0 : M.coefd[st + 1];
       AS.drift_mask = !last;
       AF.drift_mask = !last && multipole;
       FA.stage = AS.stage = st;
+      SA.disp_next = AS.disp_next = ahead && last ? dbuf[cur ^ 1] : nullptr;
+      AF.chi_next = ahead && last ? cbuf[cur ^ 1] : nullptr;
       SA.direct = 1;
       SA.cv = newmark ? 0.0 : M.coefv[st];
       SA.cd_next = newmark ? 0.0 : M.coefd[st + 1];
@@ -3815,24 +3938,27 @@ static void run_group(Runner &R, const MeshDev &M, Fields &F, Member *const *mb,
         });
       }
       AF.cv = AS.cv = newmark ? 0.0 : M.coefv[st];
-      const int nbs = (nblk(AS.npts) + kXcd - 1) / kXcd * kXcd;
-      const int nbf = M.nel_f > 0 ? nblk(AF.n) : 0;
+      AsmBlocks N{(nblk(AS.npts) + kXcd - 1) / kXcd * kXcd, M.nel_f > 0 ? nblk(AF.n) : 0, 0, 0};
       if (M.split_asm) {
+        const AsmBlocks NF{0, N.fluid, 0, 0};
         L(KC_ASM_F, [&] {
-          hipLaunchKernelGGL(k_asm<B>, dim3(nbf), dim3(256), 0, st_, AS, AF, 0);
+          hipLaunchKernelGGL(k_asm<B>, dim3(NF.fluid), dim3(256), 0, st_, AS, AF, RA, KA, NF);
         });
+        N.fluid = 0;
+      }
+      if (newmark) {
+        N.rec = any ? nblk(maxrec) : 0;
+        N.kwf = snap ? kwf_blocks : 0;
       }
       L(KC_ASM_S, [&] {
-        hipLaunchKernelGGL(k_asm<B>, dim3(nbs + (M.split_asm ? 0 : nbf)), dim3(256), 0, st_, AS, AF,
-                           nbs);
+        hipLaunchKernelGGL(k_asm<B>, dim3(N.solid + N.fluid + (N.rec + N.kwf) * B), dim3(256), 0,
+                           st_, AS, AF, RA, KA, N);
       });
     }
-    bool any = sample_all && maxrec > 0;
-    for (int b = 0; b < B && !any; b++)
-      any = mb[b]->nrec > 0 && (start[b] + step) % mb[b]->seis_it == 0;
-    if (!newmark && M.anel_full)
+    if (newmark) return;
+    if (M.anel_full)
       L(KC_MEMVAR, [&] { dispatch_anel_full<false, true, B>(M, st_, AN); });
-    if (!newmark && M.anel) {
+    if (M.anel) {
       // the receiver samples ride along as extra blocks of the update
       const int nrb = any ? nblk(maxrec) * B : 0;
       L(KC_MEMVAR, [&] { dispatch_memvar<B>(M, st_, SA, RA, nrb); });
@@ -3842,17 +3968,10 @@ static void run_group(Runner &R, const MeshDev &M, Fields &F, Member *const *mb,
       L(KC_REC, [&] {
         hipLaunchKernelGGL(k_receivers<B>, dim3(nblk(maxrec), B), dim3(256), 0, st_, RA);
       });
-    // kernel-wavefield snapshot of the step (a graph's steps all launch it;
-    // the kernel returns at once where the step is not a snapshot step)
-    bool snap = kw && KA.npt > 0 && sample_all;
-    for (int b = 0; b < B && kw && KA.npt > 0 && !snap; b++)
-      snap = (start[b] + step) % KA.strain_it == 0;
-    if (snap) {
-      KA.step.koff = koff;
+    if (snap)
       L(KC_REC, [&] {
         hipLaunchKernelGGL(k_kwf<B>, dim3(kwf_blocks, B), dim3(256), 0, st_, KA);
       });
-    }
   };
   auto reserve = [&](int step, int n) {
     for (int b = 0; b < B; b++) T.reserve(b, start[b] + step - 1, n, st_);
@@ -3874,7 +3993,7 @@ static void run_group(Runner &R, const MeshDev &M, Fields &F, Member *const *mb,
       R.gexec = nullptr;
       hipGraph_t g = nullptr;
       HIPCHECK(hipStreamBeginCapture(st_, hipStreamCaptureModeThreadLocal));
-      for (int k = 0; k < S; k++) one_step(k, true, k);
+      for (int k = 0; k < S; k++) one_step(k, S, true, k);
       hipLaunchKernelGGL(k_step_advance, dim3(1), dim3(64), 0, st_, RB.step_base, B, S);
       HIPCHECK(hipStreamEndCapture(st_, &g));
       const hipError_t rc = hipGraphInstantiate(&R.gexec, g, nullptr, nullptr, 0);
@@ -3894,9 +4013,9 @@ static void run_group(Runner &R, const MeshDev &M, Fields &F, Member *const *mb,
     }
   }
   // the rest, launched directly (koff counts from the current step base)
-  for (int k = 0; step < nsteps; step++, k++) {
+  for (int k = 0, n = nsteps - step; k < n; step++, k++) {
     reserve(step, 1);
-    one_step(k, false, step);
+    one_step(k, n, false, step);
   }
   HIPCHECK(hipGetLastError());
   HIPCHECK(hipEventRecord(R.ev1, st_));
@@ -4405,8 +4524,8 @@ void footprint(axh_ctx *ctx, size_t *mesh_bytes, size_t *wave_bytes) {
   if (d.nel_bdry)
     m += (size_t)d.nel_bdry * 5 * (3 * 4 + 8) + kMaxAxisBdry * 4 + (ns + nf + gs) * 4;
   if (d.anel) m += nel_s * (kCgStage + kCgUpd) * 16 + 2 * nel_s * d.n_sls * 8;
-  size_t w = 3 * gs * 4 * 3 + 3 * ns * 4 + 3 * kMaxAxisBdry * 4 + gs + gs * 4;
-  if (nel_f) w += 3 * gf * 4 + nf * 4 + nel_f * 4 + 200 * 4;
+  size_t w = 3 * gs * 4 * 4 + 3 * ns * 4 + 3 * kMaxAxisBdry * 4 + gs + gs * 4;
+  if (nel_f) w += 4 * gf * 4 + nf * 4 + nel_f * 4 + 200 * 4;
   if (d.anel) w += nel_s * (24 * d.n_sls + 24 + 4 + 24) * 4;
   w += (size_t)std::max(d.nelsrc, 0) * 25 * 16 + (size_t)d.num_rec * 4 + 4;
   if (const Array *a = ctx->get("stf")) w += a->count() * 4;   // device stf table

@@ -27,11 +27,11 @@ def _member(case, mesh, C, src, seed, path):
     fields = [el(w[k], so) for k in ("disp", "velo")] + \
              [el(w[k], fl) for k in ("chi", "dchi", "ddchi")]
     s, o = Solver.from_state_file(path), Oracle(path)
-    s.set_fields(*fields)
-    o.set_fields(*fields)
     if case["strain_it"]:
         s.kwf_grid(1, 3, 1, 3)
         s.set_kwf(strain_it=case["strain_it"])
+    s.set_fields(*fields)
+    o.set_fields(*fields)
     return s, o, st.dims
 
 
