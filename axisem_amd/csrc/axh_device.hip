@@ -104,6 +104,19 @@ static const char *const kClassName[KC_N] = {
     "predict", "stiffness", "fluid_assemble_update", "solid_assemble_update",
     "memvar_update", "receivers"};
 
+// A coupled solid point as the assembly reads it: the slots of the fluid point
+// on it (-1: none, or masked) with its inverse mass, and the coupling matrix of
+// each of its own copies (bit w of mask: copy w is coupled).  Coupled points
+// are numbered first, so a lane loads all this with its point's own data and
+// the fluid forces with its own forces.
+struct alignas(16) CplPoint {
+  int4 fslot;
+  float fminv;
+  int mask;
+  int pad[2];
+  float bm[4][2];
+};
+
 // Device allocations owned by one object and freed with it.
 struct DevAlloc {
   std::vector<void *> ptrs;
@@ -156,6 +169,7 @@ struct MeshDev {
   float *coef_s = nullptr, *m0_s = nullptr, *minv_s = nullptr;
   bool zero_term = false;  // the term zero_term_of(src) is +0 at every point
   int *einfo_s = nullptr, *gid_s = nullptr, *gstart_s = nullptr, *gslot_s = nullptr;
+  int4 *copies_s = nullptr, *copies_f = nullptr;  // point_copies
   // fluid
   float *coef_f = nullptr, *m0_f = nullptr, *minv_f = nullptr;
   float *gamma_s = nullptr, *gamma_f = nullptr;  // absorbing boundaries, or NULL
@@ -163,9 +177,10 @@ struct MeshDev {
   uint8_t *flags_f = nullptr;
   // coupling
   int *cpl_gs = nullptr, *cpl_gf = nullptr;
-  int *cpl_pt = nullptr;      // per solid point: the fluid point on it, or -1
+  int ncpl = 0;                 // coupled solid points: [0, ncpl)
+  CplPoint *cpl_pt = nullptr;   // theirs, where split_asm is off
   // the fluid is assembled by a launch of its own before the solid: absorbing
-  // boundaries, or coupling entries of one solid point on several fluid points
+  // boundaries, or coupled points that CplPoint does not hold
   bool split_asm = false;
   float *cpl_bm = nullptr;    // [nbdry*5][2]
   int *cpl_axb = nullptr;     // side-buffer slot of a masked axis point or -1
@@ -1896,6 +1911,7 @@ struct AsmSolidArgs {
   int npts;              // points assembled here (the others are kFlagDirect)
   int ncontig;           // pts[ip] == ip for ip < ncontig (not read there)
   const int *pts;
+  const int4 *copies;    // point_copies
   const int *gstart, *gslot;
   const uint8_t *flags;
   const float *minv;
@@ -1903,9 +1919,9 @@ struct AsmSolidArgs {
   double hdt, cv;
   const float *force;    // [3][nslot][B]
   float *velo, *acc0;    // [3][n][B]
-  int nsrc[kGroup];
-  const int *src_g[kGroup];
-  const float *src_val[kGroup];
+  const int4 *src_tab[kGroup];   // SourceTable
+  unsigned src_mul[kGroup];
+  int src_shift[kGroup];
   const float *stf[kGroup];  // NULL when the source is not added here
   StepRef step;
   int nstages, stage;
@@ -1929,14 +1945,17 @@ struct AsmSolidArgs {
   const float *cpl_bm;   // [entry][2]
   // the potential's second derivative of this stage: read (written by an
   // earlier launch) at the fluid point cpl_gf of each coupling entry, or NULL:
-  // formed here from the fluid forces of the one fluid point cpl_pt on a
-  // coupled solid point
+  // formed here from the fluid forces (cpl_pt of the first ncpl points)
   const float *ddchi;    // [nglob_f][B]
-  const int *cpl_gf, *cpl_pt;
+  const int *cpl_gf;
+  int ncpl;
+  const CplPoint *cpl_pt;
+  const float *force_f;  // [nslot_f][B]
 };
 
 struct AsmFluidArgs {
-  int n, newmark, mask_axis, mask_surface;
+  int n, newmark, mask_axis;
+  const int4 *copies;        // point_copies, none where the force is masked
   const int *gstart, *gslot;
   const uint8_t *flags;
   const float *minv;
@@ -1959,53 +1978,75 @@ struct AsmFluidArgs {
 template <int B>
 constexpr int kAsmChunk = (B >= 3 ? 2 : 4);
 
-// sum of the element forces of fluid point g (pdistsum_fluid), zero where
-// masked: kAsmChunk copies at a time (loads in flight together), summed in
-// ascending slot order from zero
+// sum of the forces of the fluid slots of c (pdistsum_fluid), from zero in
+// slot order; gslot, q1 continue a list of more than four
 template <int B>
-__device__ __forceinline__ void fluid_sum(const AsmFluidArgs &A, int g, float (&s)[B]) {
-  const uint8_t fl = A.flags[g];
-  const bool masked = (A.mask_axis && (fl & kFlagAxis)) ||
-                      (A.mask_surface && (fl & kFlagSurface));
+__device__ __forceinline__ void fluid_sum(const float *force, int4 c, const int *gslot, int q1,
+                                          float (&s)[B]) {
 #pragma unroll
   for (int b = 0; b < B; b++) s[b] = 0.0f;
-  if (masked) return;
+  int q = 0;
+  if (gslot && c.w < -1) {
+    q = -2 - c.w;
+    c.w = gslot[q++];
+  }
+  const int sl[4] = {c.x, c.y, c.z, c.w};
   constexpr int W = kAsmChunk<B>;
-  const int q1 = A.gstart[g + 1];
-  for (int q = A.gstart[g]; q < q1; q += W) {
-    int sl[W];
 #pragma unroll
-    for (int w = 0; w < W; w++) sl[w] = (q + w < q1) ? A.gslot[q + w] : -1;
+  for (int h = 0; h < 4; h += W) {
     float x[W][B];
 #pragma unroll
     for (int w = 0; w < W; w++)
-      if (sl[w] >= 0) ldv<B>(A.force + (size_t)sl[w] * B, x[w]);
+      if (sl[h + w] >= 0) ldv<B>(force + (size_t)sl[h + w] * B, x[w]);
 #pragma unroll
     for (int w = 0; w < W; w++)
-      if (sl[w] >= 0)
+      if (sl[h + w] >= 0)
 #pragma unroll
         for (int b = 0; b < B; b++) s[b] = s[b] + x[w][b];
   }
+  if (gslot)
+    for (; q < q1; q++) {
+      float x[B];
+      ldv<B>(force + (size_t)gslot[q] * B, x);
+#pragma unroll
+      for (int b = 0; b < B; b++) s[b] = s[b] + x[b];
+    }
 }
 
+// One lane's chain of dependent loads is what bounds this on small meshes (a
+// launch of 36 000 assembled points lasts as long as one of 1 000): the
+// point's record, then the forces it names, and nothing behind those.  Hence
+// the slots of the copies per point (one 16-byte load, not the range of a list
+// and then the list), the coupled points' fluid slots and matrices under the
+// point's own number, and the source values in a table addressed by it.
+//
 // The copies of a point are gathered kAsmChunk at a time with the three
 // components together, so that up to twelve loads are in flight per lane; each
 // component's sum still runs over the copies in ascending slot order from
 // zero.  The point's velocity (and acceleration, displacement) is loaded
 // before the gather for the same reason.
 template <int B>
-__device__ __forceinline__ void asm_solid_point(const AsmSolidArgs &A, const AsmFluidArgs &FA,
-                                                int ip) {
+__device__ __forceinline__ void asm_solid_point(const AsmSolidArgs &A, int ip) {
   const int g = ip < A.ncontig ? ip : A.pts[ip];
+  int4 cp = A.copies[g];
   const uint8_t fl = A.flags[g];
-  const int q0 = A.gstart[g], q1 = A.gstart[g + 1];
   const float mi = A.minv[g];
   float f2[B];
-  if ((fl & kFlagCoupled) && !A.ddchi) {
-    // as the fluid lanes of this launch form it
-    const int gf = A.cpl_pt[g];
-    fluid_sum<B>(FA, gf, f2);
-    const float mf = FA.minv[gf];
+  // (the matrices are held in registers where a group leaves room for them)
+  constexpr bool kHold = B <= 2;
+  float bm[kHold ? 4 : 1][2];
+  int cmask = 0;
+  if (g < A.ncpl) {
+    // the fluid's second derivative, as the fluid lanes of this launch form it
+    const CplPoint &P = A.cpl_pt[g];
+    cmask = P.mask;
+#pragma unroll
+    for (int w = 0; w < (kHold ? 4 : 0); w++) {
+      bm[w][0] = P.bm[w][0];
+      bm[w][1] = P.bm[w][1];
+    }
+    fluid_sum<B>(A.force_f, P.fslot, nullptr, 0, f2);
+    const float mf = P.fminv;
 #pragma unroll
     for (int b = 0; b < B; b++) f2[b] = -mf * f2[b];
   }
@@ -2033,62 +2074,92 @@ __device__ __forceinline__ void asm_solid_point(const AsmSolidArgs &A, const Asm
 #pragma unroll
     for (int b = 0; b < B; b++) s[c][b] = 0.0f;
   const size_t cstride = (size_t)A.nslot * B;
-  constexpr int W = kAsmChunk<B>;
-  for (int q = q0; q < q1; q += W) {
-    int sl[W];
+  // adds the copies in sl (from copy w0 on) to the sums; bdry_copy2solid
+  // (SOLVER/time_evol_wave.F90:1582-1611) enters the force of a coupled slot
+  // before the slot enters the sum
+  auto couple = [&](float (&x)[3][B], float bm0, float bm1) {
 #pragma unroll
-    for (int w = 0; w < W; w++) sl[w] = (q + w < q1) ? A.gslot[q + w] : -1;
+    for (int c = 0; c < 3; c++) {
+      if (!on[c] || (c == 1 && !A.dipole)) continue;
+      const float bmc = (c == 2) ? bm1 : bm0;
+#pragma unroll
+      for (int b = 0; b < B; b++) x[c][b] = x[c][b] + bmc * f2[b];
+    }
+  };
+  auto couple_slot = [&](float (&x)[3][B], int sl) {
+    const int p = A.cpl_slot[sl];
+    if (p < 0) return;
+    ldv<B>(A.ddchi + (size_t)A.cpl_gf[p] * B, f2);
+    couple(x, A.cpl_bm[2 * p], A.cpl_bm[2 * p + 1]);
+  };
+  const bool split = A.ddchi && (fl & kFlagCoupled);
+  int q = 0, q1 = 0;
+  if (cp.w < -1) {  // more than four copies: the rest of the list
+    q = -2 - cp.w;
+    q1 = A.gstart[g + 1];
+    cp.w = A.gslot[q++];
+  }
+  const int sl[4] = {cp.x, cp.y, cp.z, cp.w};
+  constexpr int W = kAsmChunk<B>;
+#pragma unroll
+  for (int h = 0; h < 4; h += W) {
     float x[W][3][B];
 #pragma unroll
     for (int w = 0; w < W; w++)
 #pragma unroll
       for (int c = 0; c < 3; c++)
-        if (sl[w] >= 0 && on[c]) ldv<B>(A.force + c * cstride + (size_t)sl[w] * B, x[w][c]);
-    if (fl & kFlagCoupled) {
-      // bdry_copy2solid (SOLVER/time_evol_wave.F90:1582-1611), added to the
-      // coupled slot's force before it enters the sum
+        if (sl[h + w] >= 0 && on[c])
+          ldv<B>(A.force + c * cstride + (size_t)sl[h + w] * B, x[w][c]);
+    if (cmask) {
 #pragma unroll
-      for (int w = 0; w < W; w++) {
-        const int p = sl[w] >= 0 ? A.cpl_slot[sl[w]] : -1;
-        if (p < 0) continue;
-        if (A.ddchi) ldv<B>(A.ddchi + (size_t)A.cpl_gf[p] * B, f2);
-        const float bm0 = A.cpl_bm[2 * p], bm1 = A.cpl_bm[2 * p + 1];
-#pragma unroll
-        for (int c = 0; c < 3; c++) {
-          if (!on[c] || (c == 1 && !A.dipole)) continue;
-          const float bmc = (c == 2) ? bm1 : bm0;
-#pragma unroll
-          for (int b = 0; b < B; b++) x[w][c][b] = x[w][c][b] + bmc * f2[b];
+      for (int w = 0; w < W; w++)
+        if (cmask & (1 << (h + w))) {
+          const float *m = kHold ? bm[kHold ? h + w : 0] : A.cpl_pt[g].bm[h + w];
+          couple(x[w], m[0], m[1]);
         }
-      }
+    }
+    if (split) {
+#pragma unroll
+      for (int w = 0; w < W; w++)
+        if (sl[h + w] >= 0) couple_slot(x[w], sl[h + w]);
     }
 #pragma unroll
     for (int w = 0; w < W; w++)
 #pragma unroll
       for (int c = 0; c < 3; c++)
-        if (sl[w] >= 0 && on[c])
+        if (sl[h + w] >= 0 && on[c])
 #pragma unroll
           for (int b = 0; b < B; b++) s[c][b] = s[c][b] + x[w][c][b];
   }
-  int si[B];
-  float stf[B];
+  for (; q < q1; q++) {
+    const int s1 = A.gslot[q];
+    float x[3][B];
 #pragma unroll
-  for (int b = 0; b < B; b++) {
-    si[b] = -1;
-    stf[b] = 0.0f;
-    if (fl & kFlagSource) stf[b] = stf_at(A.stf[b], A.step, b, A.nstages, A.stage);
-    if (stf[b] != 0.0f) {
-      const int *sg = A.src_g[b];
-      for (int k = 0; k < A.nsrc[b]; k++)
-        if (sg[k] == g) { si[b] = k; break; }
+    for (int c = 0; c < 3; c++)
+      if (on[c]) ldv<B>(A.force + c * cstride + (size_t)s1 * B, x[c]);
+    if (split) couple_slot(x, s1);
+#pragma unroll
+    for (int c = 0; c < 3; c++)
+      if (on[c])
+#pragma unroll
+        for (int b = 0; b < B; b++) s[c][b] = s[c][b] + x[c][b];
+  }
+  if (fl & kFlagSource) {
+#pragma unroll
+    for (int b = 0; b < B; b++) {
+      const float stf = stf_at(A.stf[b], A.step, b, A.nstages, A.stage);
+      if (stf == 0.0f || !A.src_tab[b]) continue;
+      const int4 e = A.src_tab[b][((unsigned)g * A.src_mul[b]) >> A.src_shift[b]];
+      if (e.x != g) continue;
+      const float val[3] = {__int_as_float(e.y), __int_as_float(e.z), __int_as_float(e.w)};
+#pragma unroll
+      for (int c = 0; c < 3; c++)
+        if (A.comps & (1 << c)) s[c][b] = s[c][b] - val[c] * stf;
     }
   }
 #pragma unroll
   for (int c = 0; c < 3; c++) {
     if (!(A.comps & (1 << c))) continue;
-#pragma unroll
-    for (int b = 0; b < B; b++)
-      if (si[b] >= 0) s[c][b] = s[c][b] - A.src_val[b][3 * si[b] + c] * stf[b];
     const size_t p = ((size_t)c * A.n + g) * B;
     float a[B];
     if (A.newmark) {
@@ -2157,7 +2228,8 @@ __device__ __forceinline__ void asm_solid_point(const AsmSolidArgs &A, const Asm
 template <int B>
 __device__ __forceinline__ void asm_fluid_point(const AsmFluidArgs &A, int g) {
   float s[B];
-  fluid_sum<B>(A, g, s);
+  const int4 cp = A.copies[g];
+  fluid_sum<B>(A.force, cp, A.gslot, cp.w < -1 ? A.gstart[g + 1] : 0, s);
   const float mi = A.minv[g];
   float d[B], dd[B], c[B];
   ldv<B>(A.dchi + (size_t)g * B, d);
@@ -2327,7 +2399,7 @@ void k_asm(AsmSolidArgs A, AsmFluidArgs F, RecArgs R, KwfArgs K, AsmBlocks N) {
   int blk = blockIdx.x;
   if (blk < N.solid) {
     const int ip = xcd_block(blk, N.solid) * 256 + threadIdx.x;
-    if (ip < A.npts) asm_solid_point<B>(A, F, ip);
+    if (ip < A.npts) asm_solid_point<B>(A, ip);
     return;
   }
   blk -= N.solid;
@@ -2496,19 +2568,23 @@ struct WaveHost {
 };
 
 // Renumber the solid points so that the points the assembly kernel handles
-// (all but kFlagDirect) come first, each class in its previous order: that
-// kernel then reads and writes one contiguous range of every per-point array,
-// and the stiffness kernel's single-copy points another.
+// (all but kFlagDirect) come first, the coupled ones before the others, each
+// class in its previous order: that kernel then reads and writes one
+// contiguous range of every per-point array, the stiffness kernel's
+// single-copy points another, and a coupled point's number is its index in
+// the coupling table (CplPoint).
 static void number_assembled_first(MeshHost &H) {
   const int n = H.nglob_s;
   std::vector<int> perm(n), inv(n);  // old -> new, new -> old
   int next = 0;
-  for (int pass = 0; pass < 2; pass++)
-    for (int g = 0; g < n; g++)
-      if (((H.flags_s[g] & kFlagDirect) != 0) == (pass == 1)) {
+  for (int pass = 0; pass < 3; pass++)
+    for (int g = 0; g < n; g++) {
+      const uint8_t f = H.flags_s[g];
+      if (((f & kFlagCoupled) ? 0 : (f & kFlagDirect) ? 2 : 1) == pass) {
         perm[g] = next;
         inv[next++] = g;
       }
+    }
   std::vector<int> gstart(n + 1, 0), gslot(H.gslot_s.size());
   std::vector<float> minv(n);
   std::vector<uint8_t> flags(n);
@@ -2971,6 +3047,20 @@ void global_numbering(const axh_ctx *ctx, int domain, int32_t *gid, int32_t *ngl
   *nglob = solid ? H.nglob_s : H.nglob_f;
 }
 
+// The slots of a point's copies, four per point: -1 past the last, and where a
+// point has more than four the fourth entry is -2 - q, q the list position of
+// the fourth copy in gslot.
+static std::vector<int4> point_copies(const std::vector<int> &gstart,
+                                      const std::vector<int> &gslot) {
+  std::vector<int4> out(gstart.size() - 1);
+  for (size_t g = 0; g < out.size(); g++) {
+    const int q0 = gstart[g], n = gstart[g + 1] - q0;
+    auto at = [&](int w) { return w < n ? gslot[q0 + w] : -1; };
+    out[g] = make_int4(at(0), at(1), at(2), n > 4 ? -2 - (q0 + 3) : at(3));
+  }
+  return out;
+}
+
 static std::shared_ptr<MeshDev> mesh_build(const axh_ctx *ctx) {
   const axh_dims &d = ctx->dims;
   MeshHost H;
@@ -3008,6 +3098,9 @@ static std::shared_ptr<MeshDev> mesh_build(const axh_ctx *ctx) {
   V.gid_s = m.upload(H.gid_s);
   V.gstart_s = m.upload(H.gstart_s);
   V.gslot_s = m.upload(H.gslot_s);
+  const std::vector<int4> copies_s = point_copies(H.gstart_s, H.gslot_s);
+  std::vector<int4> copies_f;
+  V.copies_s = m.upload(copies_s);
   V.minv_s = m.upload(H.minv_s);
   if (!H.gamma_s.empty()) V.gamma_s = m.upload(H.gamma_s);
   if (V.nel_f > 0) {
@@ -3017,6 +3110,14 @@ static std::shared_ptr<MeshDev> mesh_build(const axh_ctx *ctx) {
     V.gid_f = m.upload(H.gid_f);
     V.gstart_f = m.upload(H.gstart_f);
     V.gslot_f = m.upload(H.gslot_f);
+    // the masks of the fluid force (apply_axis_mask_scal of a multipole, the
+    // free surface of newmark2): no copies to sum
+    copies_f = point_copies(H.gstart_f, H.gslot_f);
+    for (int g = 0; g < V.nglob_f; g++)
+      if ((V.src != AXH_MONOPOLE && (H.flags_f[g] & kFlagAxis)) ||
+          (V.scheme == AXH_NEWMARK2 && (H.flags_f[g] & kFlagSurface)))
+        copies_f[g] = make_int4(-1, -1, -1, -1);
+    V.copies_f = m.upload(copies_f);
     V.minv_f = m.upload(H.minv_f);
     if (!H.gamma_f.empty()) V.gamma_f = m.upload(H.gamma_f);
     V.split_asm = V.gamma_f != nullptr;
@@ -3025,11 +3126,25 @@ static std::shared_ptr<MeshDev> mesh_build(const axh_ctx *ctx) {
   if (V.nbdry > 0) {
     V.cpl_gs = m.upload(H.cpl_gs);
     V.cpl_gf = m.upload(H.cpl_gf);
-    std::vector<int> pt(V.nglob_s, -1);
+    while (V.ncpl < V.nglob_s && (H.flags_s[V.ncpl] & kFlagCoupled)) V.ncpl++;
+    std::vector<CplPoint> pt(V.ncpl);
+    std::vector<int> fluid(V.ncpl, -1);
     for (size_t p = 0; p < H.cpl_gs.size(); p++) {
-      int &f = pt[H.cpl_gs[p]];
-      if (f >= 0 && f != H.cpl_gf[p]) V.split_asm = true;
-      f = H.cpl_gf[p];
+      const int gs = H.cpl_gs[p], gf = H.cpl_gf[p];
+      const int4 c = copies_s[gs], f = copies_f[gf];
+      CplPoint &P = pt[gs];
+      const int w = H.cpl_ss[p] == c.x ? 0 : H.cpl_ss[p] == c.y ? 1 : H.cpl_ss[p] == c.z ? 2
+                                       : H.cpl_ss[p] == c.w ? 3 : -1;
+      if (w < 0 || f.w < -1 || (fluid[gs] >= 0 && fluid[gs] != gf)) {
+        V.split_asm = true;
+        break;
+      }
+      fluid[gs] = gf;
+      P.fslot = f;
+      P.fminv = H.minv_f[gf];
+      P.mask |= 1 << w;
+      P.bm[w][0] = H.cpl_bm[2 * p];
+      P.bm[w][1] = H.cpl_bm[2 * p + 1];
     }
     V.cpl_pt = m.upload(pt);
     V.cpl_axb = m.upload(H.cpl_axb);
@@ -3066,10 +3181,10 @@ static std::shared_ptr<MeshDev> mesh_build(const axh_ctx *ctx) {
 // Source, receivers and blow-up flag of one wavefield (not interleaved).
 struct Member {
   DevAlloc mem;
-  int nsrc = 0;               // solid source points
-  std::vector<int> src_g_h;
-  int *src_g = nullptr;
-  float *src_val = nullptr;   // [nsrc][3]
+  std::vector<int> src_g_h;   // solid source points
+  int4 *src_tab = nullptr;    // SourceTable
+  unsigned src_mul = 0;
+  int src_shift = 31;
   int fluid_src = 0;
   int *srcel_f = nullptr;     // per fluid element: source slot k or -1
   float *src_fl = nullptr;    // source_term_fl (25 x 8)
@@ -3242,14 +3357,52 @@ static int seis_staging_samples(const axh_dims &d) {
   return std::max(1, std::min(total, kSeisStage));
 }
 
+// The solid source points of a wavefield by point number: entry
+// (g * mul) >> shift (32-bit product) holds {g, value s, phi, z} (as bits), or
+// -1 where no source point falls there.  The multiplier is searched so that
+// no two points share an entry: one load finds a point's source term.
+struct SourceTable {
+  std::vector<int4> entries;
+  unsigned mul = 0;
+  int shift = 31;
+  SourceTable(const std::vector<int> &g, const std::vector<float> &val) {
+    int bits = 4;
+    while ((1u << bits) < 4 * g.size()) bits++;
+    unsigned r = 0x9E3779B9u;
+    for (int tries = 0;; tries++) {
+      if (tries == 2000) {  // larger tables collide less
+        bits++;
+        tries = 0;
+      }
+      if (bits > 28) fail(AXH_ERR_UNSUPPORTED, "too many source points");
+      shift = 32 - bits;
+      mul = r | 1u;
+      r = r * 1664525u + 1013904223u;
+      entries.assign((size_t)1 << bits, make_int4(-1, 0, 0, 0));
+      bool ok = true;
+      for (size_t k = 0; k < g.size() && ok; k++) {
+        int4 &e = entries[((unsigned)g[k] * mul) >> shift];
+        ok = e.x < 0;
+        int v[3];
+        std::memcpy(v, &val[3 * k], sizeof v);
+        e = make_int4(g[k], v[0], v[1], v[2]);
+      }
+      if (ok) return;
+    }
+  }
+};
+
 static void member_build(const axh_ctx *ctx, const MeshDev &M, Member &W) {
   const axh_dims &d = ctx->dims;
   WaveHost H;
   build_wave_layout(ctx, M.gid_s_h, M.nglob_s, H);
   DevAlloc &m = W.mem;
-  W.nsrc = (int)H.src_g.size();
-  W.src_g = m.upload(H.src_g);
-  W.src_val = m.upload(H.src_val);
+  if (!H.src_g.empty()) {
+    const SourceTable T(H.src_g, H.src_val);
+    W.src_tab = m.upload(T.entries);
+    W.src_mul = T.mul;
+    W.src_shift = T.shift;
+  }
   W.fluid_src = d.fluid_src;
   if (M.nel_f > 0) {
     W.srcel_f = m.upload(H.srcel_f);
@@ -3808,17 +3961,17 @@ static void run_group(Runner &R, const MeshDev &M, Fields &F, Member *const *mb,
   // one wavefield: the assembled points are first the mesh's range
   // [0, first_direct) in order, then the group's source points beyond it
   AS.ncontig = F.B == 1 ? std::min(M.first_direct, F.nasm) : 0;
-  AS.gslot = M.gslot_s; AS.flags = F.flags_s; AS.minv = M.minv_s; AS.hdt = hdt;
+  AS.gslot = M.gslot_s; AS.copies = M.copies_s; AS.flags = F.flags_s; AS.minv = M.minv_s; AS.hdt = hdt;
   AS.gamma = M.gamma_s;
   AS.force = F.force_s; AS.velo = F.velo; AS.acc0 = F.acc0;
   AS.dt = dt; AS.hdt2 = hdt2; AS.cd0 = SA.cd0; AS.naxb = M.naxb; AS.axb_g = M.axb_g; AS.axb_val = F.axb_val;
-  AS.dipole = M.src == AXH_DIPOLE; AS.cpl_slot = M.cpl_slot_s; AS.cpl_pt = M.cpl_pt;
+  AS.dipole = M.src == AXH_DIPOLE; AS.cpl_slot = M.cpl_slot_s; AS.cpl_pt = M.cpl_pt; AS.ncpl = M.split_asm ? 0 : M.ncpl; AS.force_f = F.force_f;
   AS.cpl_bm = M.cpl_bm;
   AS.cpl_gf = M.cpl_gf;
   AS.ddchi = M.split_asm ? F.ddchi : nullptr;
   AsmFluidArgs AF{};
   AF.n = M.nglob_f; AF.newmark = newmark; AF.mask_axis = multipole;
-  AF.mask_surface = newmark; AF.gstart = M.gstart_f; AF.gslot = M.gslot_f;
+  AF.copies = M.copies_f; AF.gstart = M.gstart_f; AF.gslot = M.gslot_f;
   AF.flags = M.flags_f; AF.minv = M.minv_f; AF.hdt = hdt; AF.force = F.force_f;
   AF.gamma = M.gamma_f;
   AF.dchi = F.dchi; AF.ddchi = F.ddchi; AF.dt = dt; AF.hdt2 = hdt2; AF.cd0 = SA.cd0;
@@ -3834,7 +3987,7 @@ static void run_group(Runner &R, const MeshDev &M, Fields &F, Member *const *mb,
     PS.blow[b] = RB.blow[b]; PS.thr[b] = w.blow_thr;
     PF.blow[b] = RB.blow[b]; PF.thr[b] = w.blow_thr;
     AS.blow[b] = RB.blow[b]; AS.thr[b] = w.blow_thr;
-    AS.nsrc[b] = w.nsrc; AS.src_g[b] = w.src_g; AS.src_val[b] = w.src_val;
+    AS.src_tab[b] = w.src_tab; AS.src_mul[b] = w.src_mul; AS.src_shift[b] = w.src_shift;
     RA.nrec[b] = w.nrec; RA.rec_g[b] = w.rec_g; RA.ring[b] = RB.ring[b];
     RA.seis_it[b] = std::max(w.seis_it, 1); RA.cap[b] = RB.cap[b];
     maxrec = std::max(maxrec, w.nrec);
@@ -4518,11 +4671,12 @@ void footprint(axh_ctx *ctx, size_t *mesh_bytes, size_t *wave_bytes) {
   if (const Array *a = ctx->get("axis_solid"))
     for (size_t e = 0; e < a->count(); e++) nax += a->as<int32_t>()[e] != 0;
   size_t m = 105 * 4;
-  m += ns * nc * 4 + nel_s * 4 + nax * 50 * 4 + ns * 4 + (gs + 1) * 4 + nel_s * 25 * 4 + gs * 4;
+  m += ns * nc * 4 + nel_s * 4 + nax * 50 * 4 + ns * 4 + (gs + 1) * 4 + nel_s * 25 * 4 + gs * 20;
   if (nel_f) m += nf * 4 * 4 + nel_f * 4 + nel_f * 5 * 4 + nf * 4 + (gf + 1) * 4 + nel_f * 25 * 4 +
-                  gf * 4 + gf;
+                  gf * 20 + gf;
   if (d.nel_bdry)
-    m += (size_t)d.nel_bdry * 5 * (3 * 4 + 8) + kMaxAxisBdry * 4 + (ns + nf + gs) * 4;
+    m += (size_t)d.nel_bdry * 5 * (3 * 4 + 8) + kMaxAxisBdry * 4 + (ns + nf) * 4 +
+         (size_t)(4 * d.nel_bdry + 2) * sizeof(CplPoint);
   if (d.anel) m += nel_s * (kCgStage + kCgUpd) * 16 + 2 * nel_s * d.n_sls * 8;
   size_t w = 3 * gs * 4 * 4 + 3 * ns * 4 + 3 * kMaxAxisBdry * 4 + gs + gs * 4;
   if (nel_f) w += 4 * gf * 4 + nf * 4 + nel_f * 4 + 200 * 4;
