@@ -786,6 +786,19 @@ void k_solid(SolidArgs A, FluidArgs FA) {
   const int gp = valid ? A.gid[slot] : 0;
 
   stage_g(A.G, sG);
+  // the displacement is requested before the terms: loads return in order, so
+  // the barrier behind its LDS stores would otherwise also wait for the 15 to 26
+  // term loads, which the first products do not need (with the SLS sums
+  // requested early as well: 10 s mesh, dipole symplec4 anelastic, 8 steps
+  // 2947 -> 2824 us; 50 s mesh, newmark2, 40 steps 546 -> 531 us)
+  float ug[NCOMP][B];
+#pragma unroll
+  for (int cc = 0; cc < NCOMP; cc++) {
+    const int c = (NCOMP == 2 && cc == 1) ? 2 : cc;
+#pragma unroll
+    for (int b = 0; b < B; b++) ug[cc][b] = 0.0f;
+    if (valid) ldv<B>(A.disp + ((size_t)c * A.nglob + gp) * B, ug[cc]);
+  }
   // the lane's stiffness terms (the packed rows cover all 256 lanes), read
   // non-temporally: they are streamed once per launch (221 MB at 10 s) and
   // would otherwise evict the fields, forces and index lists that this and
@@ -797,7 +810,8 @@ void k_solid(SolidArgs A, FluidArgs FA) {
     for (int a = 0; a < NC; a++)
       cf[a] = (ZT && a == zero_term_of(SRC)) ? 0.0f : __builtin_nontemporal_load(coef + a * 256);
   }
-  gather_disp<NCOMP, B>(A, valid, gp, t, sU);
+#pragma unroll
+  for (int cc = 0; cc < NCOMP; cc++) stv<B>(sU + (size_t)cc * 256 * B + t * B, ug[cc]);
   // a single-copy point is kicked here at the end: its velocity (and, for
   // newmark2, acceleration) and inverse mass are requested now
   // (one wavefield only: for a group the extra state traffic at the end of
@@ -837,6 +851,10 @@ void k_solid(SolidArgs A, FluidArgs FA) {
       sCf[MV ? le : 0][MV ? jj : 0][3] = A.tstm1[jj] * ak;
     }
   }
+  // symplectic anelastic: the lane's SLS sum, needed after the products
+  float rs0[ANEL && MODE == 1 ? B : 1];
+  if constexpr (ANEL && MODE == 1)
+    if (valid && k < 24) ldv<B>(A.rsum + ((size_t)e * 24 + k) * B, rs0);
   __syncthreads();
 
   GRegs G;
@@ -1093,9 +1111,7 @@ void k_solid(SolidArgs A, FluidArgs FA) {
           R[k * B + b] = s;
         }
       } else {
-        float r[B];
-        ldv<B>(A.rsum + ((size_t)e * 24 + k) * B, r);
-        stv<B>(R + k * B, r);
+        if constexpr (ANEL && MODE == 1) stv<B>(R + k * B, rs0);
       }
     }
     const float *cs = A.cg_stage + (size_t)(valid ? e : 0) * (kCgStage * 4);
