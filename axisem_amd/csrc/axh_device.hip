@@ -43,6 +43,7 @@
 #include <memory>
 #include <mutex>
 #include <string>
+#include <type_traits>
 #include <vector>
 
 #include "axh_internal.h"
@@ -292,6 +293,14 @@ __device__ __forceinline__ float stf_at(const float *tab, const StepRef &r, int 
   return tab ? tab[(size_t)(step_of(r, b) - 1) * nst + st] : 0.0f;
 }
 
+// terms per point of the memory variables at all 25 points
+constexpr int kAfTerms = 12;
+enum { AF_Y = 0, AF_VSE, AF_VSX, AF_VZE, AF_VZX, AF_DSDE, AF_DZDE, AF_DSDX, AF_DZDX, AF_INVS,
+       AF_DMU, AF_DK };
+// attenuation of a kernel instance: none, coarse-grained memory variables, or
+// memory variables at all 25 points
+enum { kElastic = 0, kCoarse = 1, kFull = 2 };
+
 struct SolidArgs {
   int nel, nsls, nglob, nslot, ntile;
   const float *G, *coef, *m0;
@@ -299,11 +308,13 @@ struct SolidArgs {
   const float *cg_stage;  // [nel][5][4]
   const float *cg_upd;    // [nel][8][4]
   const double *aj_mu, *aj_k;  // [nel][nsls]
+  const float *af_terms;  // kFull: [tile][kAfTerms][256]
+  const float *af_axis;   // kFull: [nel][5][5]: Y0, V0_s_eta, V0_s_xi, V0_z_eta, V0_z_xi
   double expw[kMaxSls], tst[kMaxSls], tstm1[kMaxSls];
   const float *disp;      // [3][nglob][B]
   float *force;           // [3][nslot][B]
   float *memvar;          // [nel][nsls][6][4][B]
-  float *rsum;            // [nel][6][4][B]
+  float *rsum;            // [nel][6][4][B]; kFull: [tile][6][256][B]
   float *trm1;            // [nel][4][B]
   float *devm1;           // [nel][6][4][B]
   // points of kFlagDirect: the stiffness kernel does their assembly (one
@@ -726,8 +737,15 @@ __device__ __forceinline__ void fluid_tile(const FluidArgs &A, int tile, float *
 // solid stiffness: glob_stiffness_{mono,di,quad}_4 (SOLVER/stiffness_mono.f90:
 // 60-157, stiffness_di.f90:60-256, stiffness_quad.f90:238-412) followed by
 // glob_anel_stiffness_*_cg4 and, for newmark2, time_step_memvars_cg4.
-// MODE 0: newmark2 (memory variables read, used, updated)
+// MODE 0: newmark2 (coarse-grained memory variables read, used, updated)
 // MODE 1: symplectic stage (sums of memory variables read)
+// AN kFull (either mode): glob_anel_stiffness_*_4 (SOLVER/stiffness_mono.f90:
+// 409-507, stiffness_di.f90:604-723, stiffness_quad.f90:555-668) from the sums
+// of the memory variables over the SLS that k_anel_full keeps.  In a launch of
+// its own that subtraction read and wrote every element force (55 MB at 10 s)
+// and no point could be kicked here; 24 480 elements, dipole symplec4:
+// stiffness 15.9, forces 12.3 and assembly 10.6 us per stage before, 21.9 and 8.7
+// after.
 // One workgroup = one tile of 10 elements, one lane = one GLL point and the
 // B wavefields of the group; the lane's stiffness terms are read once.
 // ---------------------------------------------------------------------------
@@ -739,13 +757,15 @@ __device__ __forceinline__ void fluid_tile(const FluidArgs &A, int tile, float *
 // with attenuation uses it.
 // ZT: the term zero_term_of(SRC) is +0 at every point of the mesh and is not
 // read (the kernel multiplies by the same +0: the same IEEE operations).
-template <int SRC, int MODE, bool ANEL, int B, int MS = kMaxSls, bool ZT = false>
+template <int SRC, int MODE, int AN, int B, int MS = kMaxSls, bool ZT = false>
 __global__ __launch_bounds__(256, (B == 1 ? 5 : (B == 2 ? 3 : 2)))
 void k_solid(SolidArgs A, FluidArgs FA) {
   constexpr int NCOMP = (SRC == AXH_MONOPOLE) ? 2 : 3;
   constexpr int NC = (SRC == AXH_MONOPOLE) ? kNcMono
                      : (SRC == AXH_DIPOLE) ? kNcDi : kNcQuad;
   constexpr int NS = (SRC == AXH_MONOPOLE) ? 4 : 6;
+  constexpr bool ANEL = AN == kCoarse;
+  constexpr bool FULL = AN == kFull;
   constexpr bool MV = ANEL && MODE == 0;  // memory variables updated here
   __shared__ __align__(16) float sU[NCOMP * 256 * B];
   __shared__ __align__(16) float sS[NS][256 * B];
@@ -769,6 +789,8 @@ void k_solid(SolidArgs A, FluidArgs FA) {
   // ts_fac_t(jj) a_j and ts_fac_tm1(jj) a_j per element (mu, then kappa)
   __shared__ double sCf[MV ? kElemPerTile : 1][MV ? MS : 1][4];
   __shared__ __align__(16) float sG[105];
+  // kFull: the axial vectors of the anelastic forces, formed by the lanes (0, j)
+  __shared__ __align__(16) float sW[FULL ? 3 : 1][FULL ? kElemPerTile * 5 * B : 1];
 
   if ((int)blockIdx.x >= A.ntile) {  // a fluid tile, in the same LDS
     fluid_tile<B>(FA, blockIdx.x - A.ntile, sU, sS[0], sS[1], sG);
@@ -862,6 +884,26 @@ void k_solid(SolidArgs A, FluidArgs FA) {
   float acc[3][B];
   const float *U0 = sU + eb, *U1 = sU + 256 * B + eb, *U2 = sU + 2 * 256 * B + eb;
 
+  // kFull: the point's SLS sums and anelastic terms, requested once the
+  // stiffness terms are used up, so that they arrive during the second products
+  // (wider groups request them after those: held across them, a dipole group of
+  // 4 takes 184 registers and runs 2 waves per SIMD)
+  float fr[FULL ? 6 : 1][B], ft[FULL ? 5 : 1];
+  auto request_full = [&] {
+    if constexpr (FULL) {
+      const float *rs = A.rsum + ((size_t)tile * 6 * 256 + t) * B;
+#pragma unroll
+      for (int c = 0; c < 6; c++) {
+#pragma unroll
+        for (int b = 0; b < B; b++) fr[c][b] = 0.0f;
+        if (valid && (SRC != AXH_MONOPOLE || (c != 3 && c != 5)))
+          ldv<B>(rs + (size_t)c * 256 * B, fr[c]);
+      }
+      const float *tm = A.af_terms + (size_t)tile * kAfTerms * 256 + t;
+#pragma unroll
+      for (int a = 0; a < 5; a++) ft[a] = __builtin_nontemporal_load(tm + a * 256);
+    }
+  };
   if (SRC == AXH_MONOPOLE) {
     const float m1 = cf[0], m2 = cf[1], m3 = cf[2], m4 = cf[3], mw1 = cf[4],
                 m11s = cf[5], m21s = cf[6], m41s = cf[7], m12s = cf[8], m22s = cf[9],
@@ -883,6 +925,7 @@ void k_solid(SolidArgs A, FluidArgs FA) {
       sS[2][t * B + b] = m11z * X4 + m21z * X2 + m32s * X3 + m22s * X1 + m3 * us;
       sS[3][t * B + b] = m11z * X2 + m41z * X4 + m12s * X1 + m42s * X3 + m4 * us;
     }
+    if (B <= 2) request_full();
     __syncthreads();
     // axial terms with M0_w1..3
     float w1 = 0, w2 = 0, w3 = 0;
@@ -968,6 +1011,7 @@ void k_solid(SolidArgs A, FluidArgs FA) {
       sS[4][t * B + b] = m33s * X8 + m23s * X7 + m11z * X6 + m21z * X3 + m7 * u2;
       sS[5][t * B + b] = m13s * X7 + m43s * X8 + m11z * X3 + m41z * X6 + m8 * u2;
     }
+    if (B <= 2) request_full();
     __syncthreads();
     float w1 = 0, w2 = 0, w3 = 0, w4 = 0, w6 = 0, w7 = 0, w8 = 0, w9 = 0, w10 = 0;
     if (axial) {
@@ -1059,6 +1103,7 @@ void k_solid(SolidArgs A, FluidArgs FA) {
       sS[4][t * B + b] = m1phi * X5 + m2phi * X2 + m5 * tus + 2.0f * m7 * uz;        // S1phi
       sS[5][t * B + b] = m1phi * X2 + m4phi * X5 + m6 * tus + 2.0f * m8 * uz;        // S2phi
     }
+    if (B <= 2) request_full();
     __syncthreads();
     {
       float Y[6][B];
@@ -1097,6 +1142,153 @@ void k_solid(SolidArgs A, FluidArgs FA) {
     }
   }
 
+  if constexpr (FULL) {
+    // the S fields over the product buffers (dead since the barrier behind the
+    // second products), the axial vectors from the sums at (0, j)
+    constexpr int F4 = SRC == AXH_MONOPOLE ? 2 : 4;  // buffers of S_zeta, S_zxi
+    if (B > 2) request_full();
+    const float yl = ft[AF_Y], vse = ft[AF_VSE], vsx = ft[AF_VSX], vze = ft[AF_VZE],
+                vzx = ft[AF_VZX];
+    const int tb = t * B;
+    {
+      float S[6][B];
+#pragma unroll
+      for (int w = 0; w < B; w++) {
+        const float r1 = fr[0][w], r3 = fr[2][w], r4 = fr[3][w], r5 = fr[4][w], r6 = fr[5][w];
+        if (SRC == AXH_MONOPOLE) {
+          S[0][w] = vze * r1 + vse * r5;
+          S[1][w] = vzx * r1 + vsx * r5;
+          S[2][w] = 0.0f;
+          S[3][w] = 0.0f;
+        } else if (SRC == AXH_DIPOLE) {
+          S[0][w] = vze * (r1 - r6) + vse * (r5 - r4);
+          S[1][w] = vzx * (r1 - r6) + vsx * (r5 - r4);
+          S[2][w] = vze * (r1 + r6) + vse * (r5 + r4);
+          S[3][w] = vzx * (r1 + r6) + vsx * (r5 + r4);
+        } else {
+          S[0][w] = vze * r1 + vse * r5;
+          S[1][w] = vzx * r1 + vsx * r5;
+          S[2][w] = vze * r6 + vse * r4;
+          S[3][w] = vzx * r6 + vsx * r4;
+        }
+        S[4][w] = vze * r5 + vse * r3;
+        S[5][w] = vzx * r5 + vsx * r3;
+      }
+      stv<B>(&sS[0][tb], S[0]);
+      stv<B>(&sS[1][tb], S[1]);
+      if (SRC != AXH_MONOPOLE) {
+        stv<B>(&sS[2][tb], S[2]);
+        stv<B>(&sS[3][tb], S[3]);
+      }
+      stv<B>(&sS[F4][tb], S[4]);
+      stv<B>(&sS[F4 + 1][tb], S[5]);
+    }
+    if (axial && i == 0) {
+      const float *av = A.af_axis + (size_t)e * 25;
+      const float y0 = av[j], v0se = av[5 + j], v0sx = av[10 + j], v0ze = av[15 + j],
+                  v0zx = av[20 + j];
+#pragma unroll
+      for (int w = 0; w < B; w++) {
+        const float r10 = fr[0][w], r20 = fr[1][w], r30 = fr[2][w], r40 = fr[3][w],
+                    r50 = fr[4][w], r60 = fr[5][w];
+        float V1, V2, V3;
+        if (SRC == AXH_MONOPOLE) {
+          V1 = v0ze * r10 + v0se * r50 + y0 * r20;
+          V2 = v0ze * r50 + v0se * r30;
+          V3 = v0zx * r50 + v0sx * r30;
+        } else if (SRC == AXH_DIPOLE) {
+          V1 = v0ze * (r10 - r60) + v0se * (r50 - r40);
+          V2 = v0zx * (r10 - r60) + v0sx * (r50 - r40);
+          V3 = v0ze * (r10 + r60) + v0se * (r50 + r40) + y0 * 2.0f * (r20 - r60);
+        } else {
+          V1 = v0ze * r10 + y0 * (r20 - 2.0f * r60);
+          V2 = -(v0ze * r60) + y0 * (r60 - 2.0f * r20);
+          V3 = v0se * r30;
+        }
+        const int o = (le * 5 + j) * B + w;
+        sW[0][o] = V1;
+        sW[FULL ? 1 : 0][o] = V2;
+        sW[FULL ? 2 : 0][o] = V3;
+      }
+    }
+    __syncthreads();
+    if (valid) {
+      // one component after the other, each pinned before the next one's LDS
+      // reads (all six products at once hold 24 more registers at B = 4)
+      float l1[B], l2[B], l3[B];
+      {
+        float X1[B], X2[B];
+        amulv<B>(G.g, &sS[0][eb], i, j, X1);
+        mulbv<B>(&sS[1][eb], G.g2T, i, j, X2);
+#pragma unroll
+        for (int w = 0; w < B; w++) {
+          const float r2 = fr[1][w], r6 = fr[5][w];
+          l1[w] = X1[w] + X2[w];
+          if (SRC == AXH_MONOPOLE) l1[w] = l1[w] + yl * r2;
+          if (SRC == AXH_QUADPOLE) l1[w] = l1[w] + yl * (r2 - 2.0f * r6);
+          if (B > 2) pin(l1[w]);
+        }
+      }
+      if (SRC != AXH_MONOPOLE) {
+        float X3[B], X4[B];
+        amulv<B>(G.g, &sS[2][eb], i, j, X3);
+        mulbv<B>(&sS[3][eb], G.g2T, i, j, X4);
+#pragma unroll
+        for (int w = 0; w < B; w++) {
+          const float r2 = fr[1][w], r6 = fr[5][w];
+          if (SRC == AXH_DIPOLE) l2[w] = X3[w] + X4[w] + 2.0f * yl * (r2 - r6);
+          else l2[w] = -X3[w] - X4[w] + yl * (r6 - 2.0f * r2);
+          if (B > 2) pin(l2[w]);
+        }
+      }
+      {
+        float X5[B], X6[B];
+        amulv<B>(G.g, &sS[F4][eb], i, j, X5);
+        mulbv<B>(&sS[F4 + 1][eb], G.g2T, i, j, X6);
+#pragma unroll
+        for (int w = 0; w < B; w++) {
+          const float r4 = fr[3][w];
+          l3[w] = X5[w] + X6[w];
+          if (SRC == AXH_DIPOLE) l3[w] = l3[w] - yl * r4;
+          if (SRC == AXH_QUADPOLE) l3[w] = l3[w] - 2.0f * yl * r4;
+          if (B > 2) pin(l3[w]);
+        }
+      }
+      if (axial) {
+        const float g0 = G.g0i;
+        float V1[B], V2[B], V3[B], VT[B];
+        const int o = (le * 5 + j) * B;
+        ldv<B>(&sW[0][o], V1);
+        ldv<B>(&sW[FULL ? 1 : 0][o], V2);
+        ldv<B>(&sW[FULL ? 2 : 0][o], V3);
+        // vxm_4 of the axial vector along eta: monopole V3, dipole V2
+        if (SRC != AXH_QUADPOLE)
+          vmbv<B>(&sW[FULL ? (SRC == AXH_MONOPOLE ? 2 : 1) : 0][le * 5 * B], G.g2T, j, VT);
+#pragma unroll
+        for (int w = 0; w < B; w++) {
+          l1[w] = l1[w] + g0 * V1[w];
+          if (SRC == AXH_MONOPOLE) {
+            l3[w] = l3[w] + g0 * V2[w];
+            if (i == 0) l3[w] = l3[w] + VT[w];
+          } else if (SRC == AXH_DIPOLE) {
+            if (i == 0) l1[w] = l1[w] + VT[w];
+            l2[w] = l2[w] + g0 * V3[w];
+            // the z-component adds outerprod(G0, V2) (stiffness_di.f90:706-707)
+            l3[w] = l3[w] + g0 * V2[w];
+          } else {
+            l2[w] = l2[w] + g0 * V2[w];
+            l3[w] = l3[w] + g0 * V3[w];
+          }
+        }
+      }
+#pragma unroll
+      for (int w = 0; w < B; w++) {
+        acc[0][w] = acc[0][w] - l1[w];
+        if (SRC != AXH_MONOPOLE) acc[1][w] = acc[1][w] - l2[w];
+        acc[2][w] = acc[2][w] - l3[w];
+      }
+    }
+  }
   if (ANEL) {
     // sums of the memory variables over the SLS, (c, q) per lane k < 24
     float *R = &sR[le * 24 * B];
@@ -1503,46 +1695,34 @@ __global__ __launch_bounds__(256) void k_memvar(SolidArgs A, RecArgs R) {
 }
 
 // ---------------------------------------------------------------------------
-// Memory variables at all 25 points of an element (att_coarse_grained
-// false), one wavefield: the anelastic forces of glob_anel_stiffness_*_4
-// (SOLVER/stiffness_mono.f90:409-507, stiffness_di.f90:604-723,
-// stiffness_quad.f90:555-668), subtracted from the element forces the
-// stiffness kernel wrote (before the assembly adds the coupling terms, the
-// reference's order), and time_step_memvars_4 (SOLVER/attenuation.f90:210-334)
-// with the strain of compute_strain_att_el_4 (attenuation.f90:542-606).  One
-// block per solid tile, a lane per element point (i = k % 5, j = k / 5).
-// Newmark runs both parts in one launch (the update reads the displacement the
-// forces were computed from); a symplectic step runs the forces after every
-// stage and the update once after the last drift.  The update also stores the
-// sums over the SLS of the new memory variables (from zero in SLS order, the
-// sums the forces form), so the stage launches read 6 floats per point instead
-// of 6 n_sls.
+// Memory variables at all 25 points of an element (att_coarse_grained false):
+// time_step_memvars_4 (SOLVER/attenuation.f90:210-334) with the strain of
+// compute_strain_att_el_4 (attenuation.f90:542-606).  One block per solid
+// tile, a lane per element point (i = k % 5, j = k / 5), once per step: for
+// newmark2 after the stiffness launch, which reads the sums of before, for a
+// symplectic scheme after the last drift.  The update also stores the sums over
+// the SLS of the new memory variables (from zero in SLS order, the sums the
+// anelastic forces form), so the stiffness launches read 6 floats per point
+// instead of 6 n_sls.
 // ---------------------------------------------------------------------------
-constexpr int kAfTerms = 12;
-enum { AF_Y = 0, AF_VSE, AF_VSX, AF_VZE, AF_VZX, AF_DSDE, AF_DZDE, AF_DSDX, AF_DZDX, AF_INVS,
-       AF_DMU, AF_DK };
-
 struct AnelFullArgs {
-  int nel, nsls, nglob, nslot;
+  int nel, nsls, nglob;
   const float *G;         // G0 | G1 | G1T | G2 | G2T
   const float *terms;     // [tile][kAfTerms][256]
-  const float *axis;      // [nel][5][5]: Y0, V0_s_eta, V0_s_xi, V0_z_eta, V0_z_xi
   const int *einfo, *gid;
   const double *aj_mu, *aj_k;  // [nel][nsls]
   double expw[kMaxSls], tst[kMaxSls], tstm1[kMaxSls];
   const float *disp;      // [3][nglob][B]
-  float *force;           // [3][nslot][B]
   float *memvar;          // [tile][nsls][6][256][B]
   float *trm1;            // [tile][256][B]
   float *devm1;           // [tile][6][256][B]
   float *rsum;            // [tile][6][256][B]: sums over the SLS
 };
 
-template <int SRC, bool STIFF, bool UPD, int B>
+template <int SRC, int B>
 __global__ __launch_bounds__(256) void k_anel_full(AnelFullArgs A) {
   __shared__ float sG[105];
-  __shared__ float sA[6][256 * B];  // S terms (forces), then the strain's fields
-  __shared__ float sR[6][256 * B];  // sums of the memory variables
+  __shared__ float sA[5][256 * B];  // the strain's fields
   const int t = threadIdx.x, tile = blockIdx.x;
   const int le = t / 25, k = t - 25 * le;
   const int i = k % 5, j = k / 5;
@@ -1551,9 +1731,9 @@ __global__ __launch_bounds__(256) void k_anel_full(AnelFullArgs A) {
   const int eb = le * 25;  // the element's first lane
   const size_t slot = (size_t)tile * 256 + t;
   stage_g(A.G, sG);
-  const float *G0 = sG, *G1 = sG + 5, *G1T = sG + 30, *G2 = sG + 55, *G2T = sG + 80;
+  const float *G1T = sG + 30, *G2 = sG + 55, *G2T = sG + 80;
   const bool ax = valid && A.einfo[e] >= 0;
-  const float *Gs = ax ? G1 : G2, *GsT = ax ? G1T : G2T;
+  const float *GsT = ax ? G1T : G2T;
   auto term = [&](int a) {
     return valid ? A.terms[((size_t)tile * kAfTerms + a) * 256 + t] : 0.0f;
   };
@@ -1562,290 +1742,140 @@ __global__ __launch_bounds__(256) void k_anel_full(AnelFullArgs A) {
   float *const mv = A.memvar + (size_t)tile * A.nsls * mvs + (size_t)t * B;
   float *const prs = A.rsum + (size_t)tile * mvs + (size_t)t * B;
   const int tb = t * B;
-  if (STIFF) {
-    float r[6][B];
+  const int g = valid ? A.gid[slot] : 0;
+  float u1[B], u2[B], u3[B];
 #pragma unroll
-    for (int c = 0; c < 6; c++) {
-#pragma unroll
-      for (int w = 0; w < B; w++) r[c][w] = 0.0f;
-      if (valid && (SRC != AXH_MONOPOLE || (c != 3 && c != 5))) {
-        if (UPD) {
-          for (int q = 0; q < A.nsls; q++) {
-            float x[B];
-            ldv<B>(mv + q * mvs + c * cs, x);
-#pragma unroll
-            for (int w = 0; w < B; w++) r[c][w] = r[c][w] + x[w];
-          }
-        } else {
-          ldv<B>(prs + c * cs, r[c]);
-        }
-      }
-      stv<B>(&sR[c][tb], r[c]);
-    }
-    const float yl = term(AF_Y), vse = term(AF_VSE), vsx = term(AF_VSX), vze = term(AF_VZE),
-                vzx = term(AF_VZX);
-    {
-      float S[6][B];
-#pragma unroll
-      for (int w = 0; w < B; w++) {
-        const float r1 = r[0][w], r3 = r[2][w], r4 = r[3][w], r5 = r[4][w], r6 = r[5][w];
-        if (SRC == AXH_MONOPOLE) {
-          S[0][w] = vze * r1 + vse * r5;
-          S[1][w] = vzx * r1 + vsx * r5;
-          S[2][w] = 0.0f;
-          S[3][w] = 0.0f;
-        } else if (SRC == AXH_DIPOLE) {
-          S[0][w] = vze * (r1 - r6) + vse * (r5 - r4);
-          S[1][w] = vzx * (r1 - r6) + vsx * (r5 - r4);
-          S[2][w] = vze * (r1 + r6) + vse * (r5 + r4);
-          S[3][w] = vzx * (r1 + r6) + vsx * (r5 + r4);
-        } else {
-          S[0][w] = vze * r1 + vse * r5;
-          S[1][w] = vzx * r1 + vsx * r5;
-          S[2][w] = vze * r6 + vse * r4;
-          S[3][w] = vzx * r6 + vsx * r4;
-        }
-        S[4][w] = vze * r5 + vse * r3;
-        S[5][w] = vzx * r5 + vsx * r3;
-      }
-#pragma unroll
-      for (int f = 0; f < 6; f++)
-        if (SRC != AXH_MONOPOLE || (f != 2 && f != 3)) stv<B>(&sA[f][tb], S[f]);
-    }
-    __syncthreads();
-    if (valid) {
-      const float *av = A.axis + (size_t)e * 25;
-      const int p0 = eb + 5 * j;
-      float l1[B], l2[B], l3[B];
-#pragma unroll
-      for (int w = 0; w < B; w++) {
-        const int o = eb * B + w;
-        const float r2 = r[1][w], r4 = r[3][w], r6 = r[5][w];
-        const float X1 = amul<B>(Gs, &sA[0][o], i, j), X2 = mulb<B>(&sA[1][o], G2T, i, j);
-        const float X5 = amul<B>(Gs, &sA[4][o], i, j), X6 = mulb<B>(&sA[5][o], G2T, i, j);
-        if (SRC == AXH_MONOPOLE) {
-          l1[w] = X1 + X2 + yl * r2;
-          l2[w] = 0.0f;
-          l3[w] = X5 + X6;
-        } else {
-          const float X3 = amul<B>(Gs, &sA[2][o], i, j), X4 = mulb<B>(&sA[3][o], G2T, i, j);
-          if (SRC == AXH_DIPOLE) {
-            l1[w] = X1 + X2;
-            l2[w] = X3 + X4 + 2.0f * yl * (r2 - r6);
-            l3[w] = X5 + X6 - yl * r4;
-          } else {
-            l1[w] = X1 + X2 + yl * (r2 - 2.0f * r6);
-            l2[w] = -X3 - X4 + yl * (r6 - 2.0f * r2);
-            l3[w] = X5 + X6 - 2.0f * yl * r4;
-          }
-        }
-        if (ax) {
-          // the axial vectors at this lane's j, from the sums at (0, j)
-          const float y0 = av[j], v0se = av[5 + j], v0sx = av[10 + j], v0ze = av[15 + j],
-                      v0zx = av[20 + j];
-          const int q0 = p0 * B + w;
-          const float r10 = sR[0][q0], r20 = sR[1][q0], r30 = sR[2][q0], r40 = sR[3][q0],
-                      r50 = sR[4][q0], r60 = sR[5][q0];
-          const float g0 = G0[i];
-          if (SRC == AXH_MONOPOLE) {
-            const float V1 = v0ze * r10 + v0se * r50 + y0 * r20;
-            const float V2 = v0ze * r50 + v0se * r30;
-            l1[w] = l1[w] + g0 * V1;
-            l3[w] = l3[w] + g0 * V2;
-            if (i == 0) {
-              // vxm_4(V3, G2T): V3 at every point (0, kk) of the element
-              float V4 = 0.0f;
-              for (int kk = 0; kk < 5; kk++) {
-                const int pk = (eb + 5 * kk) * B + w;
-                const float V3 = av[20 + kk] * sR[4][pk] + av[10 + kk] * sR[2][pk];
-                V4 = V4 + V3 * G2T[kk + 5 * j];
-              }
-              l3[w] = l3[w] + V4;
-            }
-          } else if (SRC == AXH_DIPOLE) {
-            const float V1 = v0ze * (r10 - r60) + v0se * (r50 - r40);
-            const float V2 = v0zx * (r10 - r60) + v0sx * (r50 - r40);
-            l1[w] = l1[w] + g0 * V1;
-            if (i == 0) {
-              float V3 = 0.0f;
-              for (int kk = 0; kk < 5; kk++) {
-                const int pk = (eb + 5 * kk) * B + w;
-                const float V2k = av[20 + kk] * (sR[0][pk] - sR[5][pk]) +
-                                  av[10 + kk] * (sR[4][pk] - sR[3][pk]);
-                V3 = V3 + V2k * G2T[kk + 5 * j];
-              }
-              l1[w] = l1[w] + V3;
-            }
-            const float Vm = v0ze * (r10 + r60) + v0se * (r50 + r40) + y0 * 2.0f * (r20 - r60);
-            l2[w] = l2[w] + g0 * Vm;
-            // the z-component adds outerprod(G0, V2) (stiffness_di.f90:706-707)
-            l3[w] = l3[w] + g0 * V2;
-          } else {
-            const float Vs = v0ze * r10 + y0 * (r20 - 2.0f * r60);
-            const float Vp = -(v0ze * r60) + y0 * (r60 - 2.0f * r20);
-            const float Vz = v0se * r30;
-            l1[w] = l1[w] + g0 * Vs;
-            l2[w] = l2[w] + g0 * Vp;
-            l3[w] = l3[w] + g0 * Vz;
-          }
-        }
-      }
-      float x[B];
-      float *f0 = A.force + slot * B, *f2 = A.force + (2 * (size_t)A.nslot + slot) * B;
-      ldv<B>(f0, x);
-#pragma unroll
-      for (int w = 0; w < B; w++) x[w] = x[w] - l1[w];
-      stv<B>(f0, x);
-      if (SRC != AXH_MONOPOLE) {
-        float *f1 = A.force + ((size_t)A.nslot + slot) * B;
-        ldv<B>(f1, x);
-#pragma unroll
-        for (int w = 0; w < B; w++) x[w] = x[w] - l2[w];
-        stv<B>(f1, x);
-      }
-      ldv<B>(f2, x);
-#pragma unroll
-      for (int w = 0; w < B; w++) x[w] = x[w] - l3[w];
-      stv<B>(f2, x);
-    }
-    if (UPD) __syncthreads();  // sA is reused below
+  for (int w = 0; w < B; w++) u1[w] = u2[w] = u3[w] = 0.0f;
+  if (valid) {
+    ldv<B>(A.disp + (size_t)g * B, u1);
+    if (SRC != AXH_MONOPOLE) ldv<B>(A.disp + ((size_t)A.nglob + g) * B, u2);
+    ldv<B>(A.disp + (2 * (size_t)A.nglob + g) * B, u3);
   }
-  if (UPD) {
-    const int g = valid ? A.gid[slot] : 0;
-    float u1[B], u2[B], u3[B];
+  // fields whose gradients the strain needs (f1 = u_z throughout)
 #pragma unroll
-    for (int w = 0; w < B; w++) u1[w] = u2[w] = u3[w] = 0.0f;
-    if (valid) {
-      ldv<B>(A.disp + (size_t)g * B, u1);
-      if (SRC != AXH_MONOPOLE) ldv<B>(A.disp + ((size_t)A.nglob + g) * B, u2);
-      ldv<B>(A.disp + (2 * (size_t)A.nglob + g) * B, u3);
+  for (int w = 0; w < B; w++) {
+    if (SRC == AXH_MONOPOLE) {
+      sA[0][tb + w] = u1[w];
+      sA[1][tb + w] = u3[w];
+    } else if (SRC == AXH_DIPOLE) {
+      sA[0][tb + w] = u1[w] + u2[w];
+      sA[1][tb + w] = u3[w];
+      sA[2][tb + w] = u2[w];
+      sA[3][tb + w] = u1[w] - u2[w];
+    } else {
+      sA[0][tb + w] = u1[w];
+      sA[1][tb + w] = u3[w];
+      sA[2][tb + w] = u2[w];
+      sA[3][tb + w] = u1[w] - 2.0f * u2[w];
+      sA[4][tb + w] = u2[w] - 2.0f * u1[w];
     }
-    // fields whose gradients the strain needs (f1 = u_z throughout)
+  }
+  __syncthreads();
+  if (!valid) return;  // no barrier follows
+  const float dse = term(AF_DSDE), dze = term(AF_DZDE), dsx = term(AF_DSDX),
+              dzx = term(AF_DZDX), is = term(AF_INVS);
+  const float dm = term(AF_DMU), dk = term(AF_DK);
+  const double third = 1.0 / 3.0;
+  float str[B], sdev[6][B];
 #pragma unroll
-    for (int w = 0; w < B; w++) {
-      if (SRC == AXH_MONOPOLE) {
-        sA[0][tb + w] = u1[w];
-        sA[1][tb + w] = u3[w];
-      } else if (SRC == AXH_DIPOLE) {
-        sA[0][tb + w] = u1[w] + u2[w];
-        sA[1][tb + w] = u3[w];
-        sA[2][tb + w] = u2[w];
-        sA[3][tb + w] = u1[w] - u2[w];
-      } else {
-        sA[0][tb + w] = u1[w];
-        sA[1][tb + w] = u3[w];
-        sA[2][tb + w] = u2[w];
-        sA[3][tb + w] = u1[w] - 2.0f * u2[w];
-        sA[4][tb + w] = u2[w] - 2.0f * u1[w];
+  for (int w = 0; w < B; w++) {
+    const int o = eb * B + w;
+    // axisym_gradient_solid_el_4: d/ds and d/dz of field f at this point
+    auto grad = [&](int f, float &ds, float &dz) {
+      const float m1 = amul<B>(GsT, &sA[f][o], i, j);
+      const float m2 = mulb<B>(&sA[f][o], G2, i, j);
+      ds = dze * m1 + dzx * m2;
+      dz = dse * m1 + dsx * m2;
+    };
+    // f_over_s_solid_el_4: f/s, and d/ds on the axis (dsdf_elem_solid)
+    auto fos = [&](int f, float val) {
+      if (ax && i == 0) {
+        float ds, dz;
+        grad(f, ds, dz);
+        return ds;
       }
+      return is * val;
+    };
+    float E[6] = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
+    float b1s, b1z, b2s, b2z;
+    grad(0, b1s, b1z);
+    grad(1, b2s, b2z);
+    E[0] = b1s;
+    E[2] = b2z;
+    E[4] = b1z + b2s;
+    if (SRC == AXH_MONOPOLE) {
+      E[1] = fos(0, u1[w]);
+    } else if (SRC == AXH_DIPOLE) {
+      E[1] = 2.0f * fos(2, u2[w]);
+      float ps, pz;
+      grad(3, ps, pz);
+      const float f3 = fos(1, u3[w]);
+      E[3] = -f3 - pz;
+      E[5] = -E[1] - ps;
+    } else {
+      E[1] = fos(3, u1[w] - 2.0f * u2[w]);
+      float ps, pz;
+      grad(2, ps, pz);
+      const float f3 = fos(1, u3[w]);
+      const float f4 = fos(4, u2[w] - 2.0f * u1[w]);
+      E[3] = -(2.0f * f3) - pz;
+      E[5] = f4 - ps;
     }
-    __syncthreads();
-    if (!valid) return;  // no barrier follows
-    const float dse = term(AF_DSDE), dze = term(AF_DZDE), dsx = term(AF_DSDX),
-                dzx = term(AF_DZDX), is = term(AF_INVS);
-    const float dm = term(AF_DMU), dk = term(AF_DK);
-    const double third = 1.0 / 3.0;
-    float str[B], sdev[6][B];
+    const float tr = E[0] + E[1] + E[2];
+    str[w] = dk * tr;
 #pragma unroll
-    for (int w = 0; w < B; w++) {
-      const int o = eb * B + w;
-      // axisym_gradient_solid_el_4: d/ds and d/dz of field f at this point
-      auto grad = [&](int f, float &ds, float &dz) {
-        const float m1 = amul<B>(GsT, &sA[f][o], i, j);
-        const float m2 = mulb<B>(&sA[f][o], G2, i, j);
-        ds = dze * m1 + dzx * m2;
-        dz = dse * m1 + dsx * m2;
-      };
-      // f_over_s_solid_el_4: f/s, and d/ds on the axis (dsdf_elem_solid)
-      auto fos = [&](int f, float val) {
-        if (ax && i == 0) {
-          float ds, dz;
-          grad(f, ds, dz);
-          return ds;
-        }
-        return is * val;
-      };
-      float E[6] = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
-      float b1s, b1z, b2s, b2z;
-      grad(0, b1s, b1z);
-      grad(1, b2s, b2z);
-      E[0] = b1s;
-      E[2] = b2z;
-      E[4] = b1z + b2s;
-      if (SRC == AXH_MONOPOLE) {
-        E[1] = fos(0, u1[w]);
-      } else if (SRC == AXH_DIPOLE) {
-        E[1] = 2.0f * fos(2, u2[w]);
-        float ps, pz;
-        grad(3, ps, pz);
-        const float f3 = fos(1, u3[w]);
-        E[3] = -f3 - pz;
-        E[5] = -E[1] - ps;
-      } else {
-        E[1] = fos(3, u1[w] - 2.0f * u2[w]);
-        float ps, pz;
-        grad(2, ps, pz);
-        const float f3 = fos(1, u3[w]);
-        const float f4 = fos(4, u2[w] - 2.0f * u1[w]);
-        E[3] = -(2.0f * f3) - pz;
-        E[5] = f4 - ps;
-      }
-      const float tr = E[0] + E[1] + E[2];
-      str[w] = dk * tr;
+    for (int c = 0; c < 6; c++) sdev[c][w] = 0.0f;
 #pragma unroll
-      for (int c = 0; c < 6; c++) sdev[c][w] = 0.0f;
-#pragma unroll
-      for (int c = 0; c < 3; c++)
-        sdev[c][w] = (float)((double)(dm * 2.0f) * ((double)E[c] - (double)tr * third));
-      sdev[4][w] = dm * E[4];
-      if (SRC != AXH_MONOPOLE) {
-        sdev[3][w] = dm * E[3];
-        sdev[5][w] = dm * E[5];
-      }
+    for (int c = 0; c < 3; c++)
+      sdev[c][w] = (float)((double)(dm * 2.0f) * ((double)E[c] - (double)tr * third));
+    sdev[4][w] = dm * E[4];
+    if (SRC != AXH_MONOPOLE) {
+      sdev[3][w] = dm * E[3];
+      sdev[5][w] = dm * E[5];
     }
-    float *ptr = A.trm1 + slot * B;
-    float *pdev = A.devm1 + (size_t)tile * mvs + (size_t)t * B;
-    float trm1[B], devm1[6][B];
-    ldv<B>(ptr, trm1);
+  }
+  float *ptr = A.trm1 + slot * B;
+  float *pdev = A.devm1 + (size_t)tile * mvs + (size_t)t * B;
+  float trm1[B], devm1[6][B];
+  ldv<B>(ptr, trm1);
 #pragma unroll
-    for (int c = 0; c < 6; c++) ldv<B>(pdev + c * cs, devm1[c]);
-    const double *amu = A.aj_mu + (size_t)A.nsls * e, *akap = A.aj_k + (size_t)A.nsls * e;
-    float rs[6][B];
+  for (int c = 0; c < 6; c++) ldv<B>(pdev + c * cs, devm1[c]);
+  const double *amu = A.aj_mu + (size_t)A.nsls * e, *akap = A.aj_k + (size_t)A.nsls * e;
+  float rs[6][B];
 #pragma unroll
-    for (int c = 0; c < 6; c++)
+  for (int c = 0; c < 6; c++)
 #pragma unroll
-      for (int w = 0; w < B; w++) rs[c][w] = 0.0f;
-    for (int q = 0; q < A.nsls; q++) {
-      const double Tt = A.tst[q], Tm = A.tstm1[q], Ew = A.expw[q];
-      const double ak = akap[q], am = amu[q];
-      float trb[B];
+    for (int w = 0; w < B; w++) rs[c][w] = 0.0f;
+  for (int q = 0; q < A.nsls; q++) {
+    const double Tt = A.tst[q], Tm = A.tstm1[q], Ew = A.expw[q];
+    const double ak = akap[q], am = amu[q];
+    float trb[B];
 #pragma unroll
-      for (int w = 0; w < B; w++)
-        trb[w] = (float)(Tt * ak * (double)str[w] + Tm * ak * (double)trm1[w]);
-      float *m = mv + q * mvs;
-#pragma unroll
-      for (int c = 0; c < 6; c++) {
-        if (SRC == AXH_MONOPOLE && (c == 3 || c == 5)) continue;
-        float x[B];
-        ldv_nt<B>(m + c * cs, x);
-#pragma unroll
-        for (int w = 0; w < B; w++) {
-          const float db =
-              (float)(Tt * am * (double)sdev[c][w] + Tm * am * (double)devm1[c][w]);
-          const double old = (double)x[w];
-          x[w] = c < 3 ? (float)((Ew * old + (double)db) + (double)trb[w])
-                       : (float)(Ew * old + (double)db);
-          rs[c][w] = rs[c][w] + x[w];
-        }
-        stv_nt<B>(m + c * cs, x);
-      }
-    }
-    stv<B>(ptr, str);
+    for (int w = 0; w < B; w++)
+      trb[w] = (float)(Tt * ak * (double)str[w] + Tm * ak * (double)trm1[w]);
+    float *m = mv + q * mvs;
 #pragma unroll
     for (int c = 0; c < 6; c++) {
-      stv<B>(pdev + c * cs, sdev[c]);
-      if (!STIFF) stv<B>(prs + c * cs, rs[c]);  // read by the symplectic stages
+      if (SRC == AXH_MONOPOLE && (c == 3 || c == 5)) continue;
+      float x[B];
+      ldv_nt<B>(m + c * cs, x);
+#pragma unroll
+      for (int w = 0; w < B; w++) {
+        const float db =
+            (float)(Tt * am * (double)sdev[c][w] + Tm * am * (double)devm1[c][w]);
+        const double old = (double)x[w];
+        x[w] = c < 3 ? (float)((Ew * old + (double)db) + (double)trb[w])
+                     : (float)(Ew * old + (double)db);
+        rs[c][w] = rs[c][w] + x[w];
+      }
+      stv_nt<B>(m + c * cs, x);
     }
+  }
+  stv<B>(ptr, str);
+#pragma unroll
+  for (int c = 0; c < 6; c++) {
+    stv<B>(pdev + c * cs, sdev[c]);
+    stv<B>(prs + c * cs, rs[c]);  // read by the stiffness launches
   }
 }
 
@@ -2823,11 +2853,9 @@ static void build_mesh_layout(const axh_ctx *ctx, MeshHost &H) {
   // ---- points with a single element copy and nothing else to add (no axis
   // mask, no coupling term; source points are excluded when a wavefield with
   // a source there is attached) ----
-  // (none with memory variables at all points: the stiffness kernel would
-  // kick them before the anelastic forces are subtracted)
   const bool anel_full = d.anel && !d.coarse_grained;
   for (int g = 0; g < H.nglob_s; g++)
-    if (!absorbing && !anel_full && H.gstart_s[g + 1] - H.gstart_s[g] == 1 &&
+    if (!absorbing && H.gstart_s[g + 1] - H.gstart_s[g] == 1 &&
         !(H.flags_s[g] & (kFlagAxis | kFlagCoupled)))
       H.flags_s[g] |= kFlagDirect;
   number_assembled_first(H);
@@ -3806,54 +3834,54 @@ struct Launcher {
 
 // one launch: the solid tiles, then the fluid tiles (the Newmark
 // memory-variable update sized for 5 linear solids where that suffices)
-template <int SRC, int MODE, bool ANEL, int B>
+template <int SRC, int MODE, int AN, int B>
 static void launch_solid(const MeshDev &M, hipStream_t s, const SolidArgs &A,
                          const FluidArgs &F) {
   const int nblocks = M.ntile_s + (M.nel_f > 0 ? M.ntile_f : 0);
+  auto launch = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, dim3(nblocks), dim3(256), 0, s, A, F);
+  };
+  auto sized = [&](auto zt) {
+    constexpr bool ZT = decltype(zt)::value;
+    if constexpr (MODE == 0 && AN == kCoarse) {
+      if (M.nsls <= 5) return launch(k_solid<SRC, MODE, AN, B, 5, ZT>);
+    }
+    launch(k_solid<SRC, MODE, AN, B, kMaxSls, ZT>);
+  };
   if constexpr (B == 1 && zero_term_of(SRC) >= 0) {
     // one wavefield of an isotropic model: the +0 term is not read (a group's
     // launch is bound by instruction issue, not by the term bytes)
-    if (M.zero_term) {
-      if (MODE == 0 && ANEL && M.nsls <= 5)
-        hipLaunchKernelGGL((k_solid<SRC, MODE, ANEL, 1, 5, true>), dim3(nblocks), dim3(256), 0,
-                           s, A, F);
-      else
-        hipLaunchKernelGGL((k_solid<SRC, MODE, ANEL, 1, kMaxSls, true>), dim3(nblocks),
-                           dim3(256), 0, s, A, F);
-      return;
-    }
+    if (M.zero_term) return sized(std::true_type{});
   }
-  if (MODE == 0 && ANEL && M.nsls <= 5)
-    hipLaunchKernelGGL((k_solid<SRC, MODE, ANEL, B, 5>), dim3(nblocks), dim3(256), 0, s, A, F);
-  else
-    hipLaunchKernelGGL((k_solid<SRC, MODE, ANEL, B>), dim3(nblocks), dim3(256), 0, s, A, F);
+  sized(std::false_type{});
 }
 
 template <int B>
 static void dispatch_solid(const MeshDev &M, hipStream_t s, const SolidArgs &A,
                            const FluidArgs &F, int mode) {
-  const bool an = M.anel != 0;
-#define AXH_SOLID_CASE(S)                                                              \
-  if (mode == 0) {                                                                     \
-    if (an) launch_solid<S, 0, true, B>(M, s, A, F); else launch_solid<S, 0, false, B>(M, s, A, F); \
-  } else {                                                                             \
-    if (an) launch_solid<S, 1, true, B>(M, s, A, F); else launch_solid<S, 1, false, B>(M, s, A, F); \
-  }
+  const int an = M.anel ? kCoarse : M.anel_full ? kFull : kElastic;
+#define AXH_SOLID_MODE(S, MODE)                                         \
+  if (an == kCoarse) launch_solid<S, MODE, kCoarse, B>(M, s, A, F);     \
+  else if (an == kFull) launch_solid<S, MODE, kFull, B>(M, s, A, F);    \
+  else launch_solid<S, MODE, kElastic, B>(M, s, A, F);
+#define AXH_SOLID_CASE(S) \
+  if (mode == 0) { AXH_SOLID_MODE(S, 0) } else { AXH_SOLID_MODE(S, 1) }
   if (M.src == AXH_MONOPOLE) { AXH_SOLID_CASE(AXH_MONOPOLE) }
   else if (M.src == AXH_DIPOLE) { AXH_SOLID_CASE(AXH_DIPOLE) }
   else { AXH_SOLID_CASE(AXH_QUADPOLE) }
 #undef AXH_SOLID_CASE
+#undef AXH_SOLID_MODE
 }
 
-template <bool STIFF, bool UPD, int B>
+template <int B>
 static void dispatch_anel_full(const MeshDev &M, hipStream_t s, const AnelFullArgs &A) {
   const dim3 grid(M.ntile_s), blk(256);
   if (M.src == AXH_MONOPOLE)
-    hipLaunchKernelGGL((k_anel_full<AXH_MONOPOLE, STIFF, UPD, B>), grid, blk, 0, s, A);
+    hipLaunchKernelGGL((k_anel_full<AXH_MONOPOLE, B>), grid, blk, 0, s, A);
   else if (M.src == AXH_DIPOLE)
-    hipLaunchKernelGGL((k_anel_full<AXH_DIPOLE, STIFF, UPD, B>), grid, blk, 0, s, A);
+    hipLaunchKernelGGL((k_anel_full<AXH_DIPOLE, B>), grid, blk, 0, s, A);
   else
-    hipLaunchKernelGGL((k_anel_full<AXH_QUADPOLE, STIFF, UPD, B>), grid, blk, 0, s, A);
+    hipLaunchKernelGGL((k_anel_full<AXH_QUADPOLE, B>), grid, blk, 0, s, A);
 }
 
 // the SLS capacity of the kernel: 5 (the reference's default number of
@@ -3928,6 +3956,7 @@ static void run_group(Runner &R, const MeshDev &M, Fields &F, Member *const *mb,
   SA.nel = M.nel_s; SA.nsls = M.nsls; SA.nglob = M.nglob_s; SA.nslot = (int)nslot_s;
   SA.ntile = M.ntile_s;
   SA.G = M.G; SA.coef = M.coef_s; SA.m0 = M.m0_s; SA.einfo = M.einfo_s; SA.gid = M.gid_s;
+  SA.af_terms = M.af_terms; SA.af_axis = M.af_axis;
   SA.cg_stage = M.cg_stage; SA.cg_upd = M.cg_upd; SA.aj_mu = M.aj_mu; SA.aj_k = M.aj_k;
   for (int s = 0; s < kMaxSls; s++) {
     SA.expw[s] = M.expw[s]; SA.tst[s] = M.tst[s]; SA.tstm1[s] = M.tstm1[s];
@@ -3944,13 +3973,13 @@ static void run_group(Runner &R, const MeshDev &M, Fields &F, Member *const *mb,
   SA.blow = RB.blow[0]; SA.thr = mb[0]->blow_thr;
   AnelFullArgs AN{};
   if (M.anel_full) {
-    AN.nel = M.nel_s; AN.nsls = M.nsls; AN.nglob = M.nglob_s; AN.nslot = (int)nslot_s;
-    AN.G = M.G; AN.terms = M.af_terms; AN.axis = M.af_axis; AN.einfo = M.einfo_s;
+    AN.nel = M.nel_s; AN.nsls = M.nsls; AN.nglob = M.nglob_s;
+    AN.G = M.G; AN.terms = M.af_terms; AN.einfo = M.einfo_s;
     AN.gid = M.gid_s; AN.aj_mu = M.aj_mu; AN.aj_k = M.aj_k;
     for (int s = 0; s < kMaxSls; s++) {
       AN.expw[s] = M.expw[s]; AN.tst[s] = M.tst[s]; AN.tstm1[s] = M.tstm1[s];
     }
-    AN.force = F.force_s; AN.memvar = F.memvar; AN.trm1 = F.trm1;
+    AN.memvar = F.memvar; AN.trm1 = F.trm1;
     AN.devm1 = F.devm1; AN.rsum = F.rsum;
   }
   FluidArgs FA{};
@@ -4099,13 +4128,6 @@ static void run_group(Runner &R, const MeshDev &M, Fields &F, Member *const *mb,
       SA.cd_next = newmark ? 0.0 : M.coefd[st + 1];
       L(KC_SOLID, [&] { dispatch_solid<B>(M, st_, SA, FA, newmark ? 0 : 1); });
       SA.direct = 0;
-      if (M.anel_full) {
-        // anelastic forces; Newmark also updates the memory variables here
-        L(KC_MEMVAR, [&] {
-          if (newmark) dispatch_anel_full<true, true, B>(M, st_, AN);
-          else dispatch_anel_full<true, false, B>(M, st_, AN);
-        });
-      }
       AF.cv = AS.cv = newmark ? 0.0 : M.coefv[st];
       AsmBlocks N{(nblk(AS.npts) + kXcd - 1) / kXcd * kXcd, M.nel_f > 0 ? nblk(AF.n) : 0, 0, 0};
       if (M.split_asm) {
@@ -4124,9 +4146,8 @@ static void run_group(Runner &R, const MeshDev &M, Fields &F, Member *const *mb,
                            st_, AS, AF, RA, KA, N);
       });
     }
+    if (M.anel_full) L(KC_MEMVAR, [&] { dispatch_anel_full<B>(M, st_, AN); });
     if (newmark) return;
-    if (M.anel_full)
-      L(KC_MEMVAR, [&] { dispatch_anel_full<false, true, B>(M, st_, AN); });
     if (M.anel) {
       // the receiver samples ride along as extra blocks of the update
       const int nrb = any ? nblk(maxrec) * B : 0;
