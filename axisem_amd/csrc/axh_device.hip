@@ -1719,10 +1719,20 @@ struct AnelFullArgs {
   float *rsum;            // [tile][6][256][B]: sums over the SLS
 };
 
-template <int SRC, int B>
+// What bounds it: 9.2 KB per element of memory variables, sources and sums, so
+// the loads in flight.  The components run outside and the SLS (MS >= n_sls)
+// inside: a component then needs its own sources only, not all six as doubles
+// (dipole group of 4: 244 -> 140 VGPRs, 2 -> 3 waves per SIMD), and its memory
+// variables of every SLS are requested together; one wavefield requests all of
+// them before the displacement, two request one component ahead.  24 480
+// elements, dipole: 42.9 -> 37 us (6.1 TB/s); whole steps: 2 monopoles 883 -> 824
+// us, monopole newmark2 761 -> 718 us, group of 4 dipoles 1757 -> 1739 us.
+template <int SRC, int B, int MS>
 __global__ __launch_bounds__(256) void k_anel_full(AnelFullArgs A) {
   __shared__ float sG[105];
   __shared__ float sA[5][256 * B];  // the strain's fields
+  // ts_fac_t(q) a_j, ts_fac_tm1(q) a_j per element (mu, then kappa)
+  __shared__ double sCf[kElemPerTile][MS][4];
   const int t = threadIdx.x, tile = blockIdx.x;
   const int le = t / 25, k = t - 25 * le;
   const int i = k % 5, j = k / 5;
@@ -1750,6 +1760,30 @@ __global__ __launch_bounds__(256) void k_anel_full(AnelFullArgs A) {
     ldv<B>(A.disp + (size_t)g * B, u1);
     if (SRC != AXH_MONOPOLE) ldv<B>(A.disp + ((size_t)A.nglob + g) * B, u2);
     ldv<B>(A.disp + (2 * (size_t)A.nglob + g) * B, u3);
+  }
+  // the memory variables of component c, all SLS
+  constexpr bool kAhead = B <= 2;
+  constexpr bool kAll = B == 1;
+  float nx[kAll ? 6 : 1][MS][B];
+  auto request = [&](int c) {
+#pragma unroll
+    for (int q = 0; q < MS; q++)
+      if (q < A.nsls) ldv_nt<B>(mv + q * mvs + c * cs, nx[kAll ? c : 0][q]);
+  };
+  if (valid && kAhead) {
+    request(0);
+    if (kAll) {
+#pragma unroll
+      for (int c = 1; c < 6; c++)
+        if (SRC != AXH_MONOPOLE || (c != 3 && c != 5)) request(c);
+    }
+  }
+  if (valid && k < A.nsls) {
+    const double am = A.aj_mu[(size_t)A.nsls * e + k], ak = A.aj_k[(size_t)A.nsls * e + k];
+    sCf[le][k][0] = A.tst[k] * am;
+    sCf[le][k][1] = A.tstm1[k] * am;
+    sCf[le][k][2] = A.tst[k] * ak;
+    sCf[le][k][3] = A.tstm1[k] * ak;
   }
   // fields whose gradients the strain needs (f1 = u_z throughout)
 #pragma unroll
@@ -1833,49 +1867,63 @@ __global__ __launch_bounds__(256) void k_anel_full(AnelFullArgs A) {
       sdev[3][w] = dm * E[3];
       sdev[5][w] = dm * E[5];
     }
+    if (B > 1) {  // one wavefield's strain after the other
+      pin(str[w]);
+#pragma unroll
+      for (int c = 0; c < 6; c++) pin(sdev[c][w]);
+    }
   }
   float *ptr = A.trm1 + slot * B;
   float *pdev = A.devm1 + (size_t)tile * mvs + (size_t)t * B;
-  float trm1[B], devm1[6][B];
-  ldv<B>(ptr, trm1);
+  float trb[MS][B];
+  {
+    float trm1[B];
+    ldv<B>(ptr, trm1);
 #pragma unroll
-  for (int c = 0; c < 6; c++) ldv<B>(pdev + c * cs, devm1[c]);
-  const double *amu = A.aj_mu + (size_t)A.nsls * e, *akap = A.aj_k + (size_t)A.nsls * e;
-  float rs[6][B];
+    for (int q = 0; q < MS; q++) {
+      if (q >= A.nsls) break;
+      const double *cf = sCf[le][q];
 #pragma unroll
-  for (int c = 0; c < 6; c++)
-#pragma unroll
-    for (int w = 0; w < B; w++) rs[c][w] = 0.0f;
-  for (int q = 0; q < A.nsls; q++) {
-    const double Tt = A.tst[q], Tm = A.tstm1[q], Ew = A.expw[q];
-    const double ak = akap[q], am = amu[q];
-    float trb[B];
-#pragma unroll
-    for (int w = 0; w < B; w++)
-      trb[w] = (float)(Tt * ak * (double)str[w] + Tm * ak * (double)trm1[w]);
-    float *m = mv + q * mvs;
-#pragma unroll
-    for (int c = 0; c < 6; c++) {
-      if (SRC == AXH_MONOPOLE && (c == 3 || c == 5)) continue;
-      float x[B];
-      ldv_nt<B>(m + c * cs, x);
-#pragma unroll
-      for (int w = 0; w < B; w++) {
-        const float db =
-            (float)(Tt * am * (double)sdev[c][w] + Tm * am * (double)devm1[c][w]);
-        const double old = (double)x[w];
-        x[w] = c < 3 ? (float)((Ew * old + (double)db) + (double)trb[w])
-                     : (float)(Ew * old + (double)db);
-        rs[c][w] = rs[c][w] + x[w];
-      }
-      stv_nt<B>(m + c * cs, x);
+      for (int w = 0; w < B; w++)
+        trb[q][w] = (float)(cf[2] * (double)str[w] + cf[3] * (double)trm1[w]);
     }
+    stv<B>(ptr, str);
   }
-  stv<B>(ptr, str);
 #pragma unroll
   for (int c = 0; c < 6; c++) {
+    // a monopole's components 3 and 5 are not updated and sum to zero
+    const bool off = SRC == AXH_MONOPOLE && (c == 3 || c == 5);
+    float rs[B];
+#pragma unroll
+    for (int w = 0; w < B; w++) rs[w] = 0.0f;
+    if (!off) {
+      float x[MS][B], od[B];
+      if (!kAhead) request(c);
+      ldv<B>(pdev + c * cs, od);
+#pragma unroll
+      for (int q = 0; q < MS; q++)
+#pragma unroll
+        for (int w = 0; w < B; w++) x[q][w] = nx[kAll ? c : 0][q][w];
+      const int next = SRC == AXH_MONOPOLE && c == 2 ? 4 : c + 1;
+      if (kAhead && !kAll && next < 6 && !(SRC == AXH_MONOPOLE && next == 5)) request(next);
+#pragma unroll
+      for (int q = 0; q < MS; q++) {
+        if (q >= A.nsls) break;
+        const double Ew = A.expw[q];
+        const double *cf = sCf[le][q];
+#pragma unroll
+        for (int w = 0; w < B; w++) {
+          const float db = (float)(cf[0] * (double)sdev[c][w] + cf[1] * (double)od[w]);
+          const double old = (double)x[q][w];
+          x[q][w] = c < 3 ? (float)((Ew * old + (double)db) + (double)trb[q][w])
+                          : (float)(Ew * old + (double)db);
+          rs[w] = rs[w] + x[q][w];
+        }
+        stv_nt<B>(mv + q * mvs + c * cs, x[q]);
+      }
+    }
     stv<B>(pdev + c * cs, sdev[c]);
-    stv<B>(prs + c * cs, rs[c]);  // read by the stiffness launches
+    stv<B>(prs + c * cs, rs);  // read by the stiffness launches
   }
 }
 
@@ -3873,15 +3921,20 @@ static void dispatch_solid(const MeshDev &M, hipStream_t s, const SolidArgs &A,
 #undef AXH_SOLID_MODE
 }
 
-template <int B>
-static void dispatch_anel_full(const MeshDev &M, hipStream_t s, const AnelFullArgs &A) {
+template <int B, int MS>
+static void dispatch_anel_full_ms(const MeshDev &M, hipStream_t s, const AnelFullArgs &A) {
   const dim3 grid(M.ntile_s), blk(256);
   if (M.src == AXH_MONOPOLE)
-    hipLaunchKernelGGL((k_anel_full<AXH_MONOPOLE, B>), grid, blk, 0, s, A);
+    hipLaunchKernelGGL((k_anel_full<AXH_MONOPOLE, B, MS>), grid, blk, 0, s, A);
   else if (M.src == AXH_DIPOLE)
-    hipLaunchKernelGGL((k_anel_full<AXH_DIPOLE, B>), grid, blk, 0, s, A);
+    hipLaunchKernelGGL((k_anel_full<AXH_DIPOLE, B, MS>), grid, blk, 0, s, A);
   else
-    hipLaunchKernelGGL((k_anel_full<AXH_QUADPOLE, B>), grid, blk, 0, s, A);
+    hipLaunchKernelGGL((k_anel_full<AXH_QUADPOLE, B, MS>), grid, blk, 0, s, A);
+}
+template <int B>
+static void dispatch_anel_full(const MeshDev &M, hipStream_t s, const AnelFullArgs &A) {
+  if (M.nsls <= 5) dispatch_anel_full_ms<B, 5>(M, s, A);
+  else dispatch_anel_full_ms<B, kMaxSls>(M, s, A);
 }
 
 // the SLS capacity of the kernel: 5 (the reference's default number of
