@@ -149,3 +149,27 @@ def test_convolve_traces_equals_the_formula():
     ref2 = _convolve_direct(seis.T.copy(), np.resize(stf, nt + 40).astype(np.float32), dt,
                             scale).T
     np.testing.assert_array_equal(out2, ref2)
+
+
+@pytest.mark.parametrize("nt,ntr,nj", [(1, 1, 0), (1, 3, 5), (5, 2, 3), (1023, 1, 4), (1024, 2, 401),
+                                       (1025, 3, 513), (2049, 1, 1030), (1500, 181, 30),
+                                       (2100, 543, 9), (300000, 1, 6)])
+def test_convolve_traces_tiles_and_pieces(nt, ntr, nj):
+    """Samples and terms around the tile sizes, arrays below and above the size
+    whose transfers go in pieces, and an output over its input."""
+    print("convolution of %d traces of %d samples, %d terms" % (ntr, nt, nj), flush=True)
+    rng = np.random.default_rng(nt + nj)
+    seis = (rng.standard_normal((ntr, nt)) * 1e-7).astype(np.float32)
+    seis[:, ::11] = -0.0
+    stf = (rng.standard_normal(max(nj, 1)) * 0.03).astype(np.float32)
+    L = S.library()
+    out = np.full_like(seis, 7)
+    S._check(L.axh_convolve_traces(nt, ntr, S._p(seis), nj, S._p(stf), 0.1, 1.5, S._p(out)))
+    acc = np.zeros_like(seis)
+    for j in range(1, min(nj, nt - 1) + 1):
+        p = (seis[:, :-j] * stf[j - 1]).astype(np.float64) * 0.1
+        acc[:, j:] = (acc[:, j:].astype(np.float64) + p).astype(np.float32)
+    ref = (acc.astype(np.float64) * 1.5).astype(np.float32)
+    assert np.array_equal(out.view(np.int32), ref.view(np.int32))
+    S._check(L.axh_convolve_traces(nt, ntr, S._p(seis), nj, S._p(stf), 0.1, 1.5, S._p(seis)))
+    assert np.array_equal(seis.view(np.int32), ref.view(np.int32))
