@@ -3788,8 +3788,10 @@ struct BatchState {
   std::vector<std::unique_ptr<Fields>> groups;
   std::vector<std::vector<int>> index;          // members of each group
   std::vector<std::shared_ptr<MeshDev>> mesh;   // each group's mesh part
-  Runner run;                                   // attach / detach copies
-  std::vector<std::unique_ptr<Runner>> runs;    // each group's stream
+  // each group's stream, also of its attach and detach copies: a stream more than
+  // the groups would share one of the process's four hardware queues with a
+  // group, whose launches then wait for another's
+  std::vector<std::unique_ptr<Runner>> runs;
 };
 
 void device_build(axh_ctx *ctx) {
@@ -3849,7 +3851,6 @@ void batch_attach(axh_batch *bt) {
   if (bt->state) return;
   const std::vector<axh_ctx *> &members = bt->members;
   std::unique_ptr<BatchState, BatchStateDeleter> S(new BatchState);
-  S->run.init();
   const int width = std::max(1, std::min(bt->group_width, kGroup));
   for (int type = AXH_MONOPOLE; type <= AXH_QUADPOLE; type++) {
     std::vector<int> of_type;
@@ -3887,20 +3888,20 @@ void batch_attach(axh_batch *bt) {
         srcs.push_back(&members[of_type[next + b]]->dev->member.src_g_h);
       fields_set_sources(*mesh, *F, srcs);
       std::vector<int> idx;
+      S->runs.emplace_back(new Runner);
+      S->runs.back()->init();
       for (int b = 0; b < size; b++, next++) {
         Device &D = *members[of_type[next]]->dev;
         if (D.run.stream) HIPCHECK(hipStreamSynchronize(D.run.stream));
-        copy_state(*mesh, *F, b, D.own, 0, S->run.stream);
+        copy_state(*mesh, *F, b, D.own, 0, S->runs.back()->stream);
         idx.push_back(of_type[next]);
       }
       S->index.push_back(idx);
       S->groups.push_back(std::move(F));
       S->mesh.push_back(mesh);
-      S->runs.emplace_back(new Runner);
-      S->runs.back()->init();
     }
   }
-  HIPCHECK(hipStreamSynchronize(S->run.stream));
+  for (auto &r : S->runs) HIPCHECK(hipStreamSynchronize(r->stream));
   for (size_t g = 0; g < S->groups.size(); g++)
     for (size_t b = 0; b < S->index[g].size(); b++) {
       Device &D = *members[S->index[g][b]]->dev;
@@ -3919,14 +3920,18 @@ void batch_detach(axh_batch *bt) {
     for (size_t b = 0; b < S.index[g].size(); b++) {
       Device &D = *bt->members[S.index[g][b]]->dev;
       try {
-        copy_state(*D.mesh, D.own, 0, *S.groups[g], (int)b, S.run.stream);
+        copy_state(*D.mesh, D.own, 0, *S.groups[g], (int)b, S.runs[g]->stream);
       } catch (const Error &e) {
         err = e.msg;
       }
       D.live = nullptr;
       D.live_slot = 0;
     }
-  const hipError_t rc = hipStreamSynchronize(S.run.stream);
+  hipError_t rc = hipSuccess;
+  for (auto &r : S.runs) {
+    const hipError_t q = hipStreamSynchronize(r->stream);
+    if (q != hipSuccess) rc = q;
+  }
   bt->state.reset();
   if (!err.empty()) fail(AXH_ERR_HIP, err);
   if (rc != hipSuccess) fail(AXH_ERR_HIP, std::string("batch detach: ") + hipGetErrorString(rc));
