@@ -3548,6 +3548,7 @@ struct Runner {
   hipStream_t stream = nullptr;
   hipEvent_t ev0 = nullptr, ev1 = nullptr;
   bool profile = false;
+  bool alone = true;   // no other group's launches are queued beside these
   std::vector<hipEvent_t> kev;  // pairs
   std::vector<int> kev_class;
   double kms[KC_N] = {0};
@@ -4062,6 +4063,7 @@ struct KwfLaunch {
   KwfTail *tail[kGroup] = {};
 };
 constexpr int kKwfBlocks = 1024;   // grid of k_kwf (grid-stride over the points)
+constexpr int kReplayLaunches = 40;  // fewest launches of a graph that is replayed
 
 template <int B>
 static void run_group(Runner &R, const MeshDev &M, Fields &F, Member *const *mb,
@@ -4305,7 +4307,16 @@ static void run_group(Runner &R, const MeshDev &M, Fields &F, Member *const *mb,
 
   int step = 0;
   const int S = R.graph_steps;
-  bool fits = S > 0 && !R.profile && nsteps >= S;
+  // A replay also predicts its first step and advances the step base (10 us on the
+  // 50 s mesh, 16 on 1200 x 160 elements), and saves 0.25 to 0.5 us per launch
+  // where kernels are short.  50 s mesh, replayed / direct: newmark2 in graphs of
+  // 4 steps (8 launches) 550 / 486 us, of 20 (40) 463 / 486; symplec4 anelastic of
+  // 4 (36) 1042 / 1042, of 8 (72) 1004 / 1042.  10 s mesh, of 4 (36) 2797 / 2748;
+  // kernel wavefields, of 2 (4) 1295 / 1190.  Groups queued beside others replay
+  // (the host is then what the others wait for: three groups of the 20 s mesh,
+  // 8 steps, 597 / 631).
+  const int launches = S * (M.nstages * (M.split_asm ? 3 : 2) + (M.anel || M.anel_full ? 1 : 0));
+  bool fits = S > 0 && !R.profile && nsteps >= S && (!R.alone || launches >= kReplayLaunches);
   for (int b = 0; b < B && fits; b++)
     fits = mb[b]->nrec <= 0 || S / std::max(mb[b]->seis_it, 1) + 1 <= RB.cap[b];
   if (kw) fits = fits && S / kw->args.strain_it + 1 <= kw->args.cap;
@@ -4604,6 +4615,7 @@ void batch_run(axh_batch *bt, int32_t nsteps, float *const *seis, float *const *
     Runner &R = *S.runs[g];
     R.profile = bt->profile;
     R.graph_steps = bt->graph_steps;
+    R.alone = S.groups.size() == 1;
     const std::vector<int> &idx = S.index[g];
     const MeshDev &M = *S.mesh[g];
     Member *mb[kGroup];

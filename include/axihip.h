@@ -286,7 +286,8 @@ int axh_kernel_stats(const axh_ctx *ctx, int kclass, double *total_ms,
 /* Launch mode of axh_run: steps = 0 launches every kernel directly (the
  * default); steps = S > 0 captures S time steps of the context once into a
  * HIP graph and replays it for every S steps of a run (the rest of a run,
- * and runs with per-kernel profiling on, launch directly).  Each kernel reads
+ * runs with per-kernel profiling on, and runs that are faster so -- one group
+ * and a graph of fewer than 40 launches -- launch directly).  Each kernel reads
  * its time step from device memory, so the replays need no host work per
  * step; results are bit-identical either way.  Small meshes, whose steps are
  * bound by launch latency, gain.  The reference has no counterpart (its time
