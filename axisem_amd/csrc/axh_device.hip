@@ -1947,6 +1947,10 @@ struct PredArgs {
   int *blow[kGroup];
   double thr[kGroup];
   StepRef step;
+  // the first launch of a run: step base, first steps and clock (NULL: not it)
+  int *set_base;
+  int first[kGroup];
+  uint64_t *set_clock;
 };
 
 template <int B>
@@ -1961,7 +1965,8 @@ __device__ __forceinline__ void predict_point(const PredArgs &A, int g) {
     if (A.check_blow && (fl & kFlagBlow)) {
 #pragma unroll
       for (int b = 0; b < B; b++)
-        if ((double)fabsf(u[b]) > A.thr[b]) atomicMin(A.blow[b], step_of(A.step, b));
+        if ((double)fabsf(u[b]) > A.thr[b])
+          atomicMin(A.blow[b], A.set_base ? A.first[b] : step_of(A.step, b));
     }
     if (A.newmark) {
       float a0[B];
@@ -1989,6 +1994,11 @@ __device__ __forceinline__ void predict_point(const PredArgs &A, int g) {
 // workgroups take the solid points, the others the fluid points.
 template <int B>
 __global__ __launch_bounds__(256) void k_predict(PredArgs S, PredArgs F, int nblk_s) {
+  if (S.set_base && blockIdx.x == 0 && threadIdx.x < B) {
+    // (no lane of this launch reads the base)
+    S.set_base[threadIdx.x] = S.first[threadIdx.x];
+    if (threadIdx.x == 0) *S.set_clock = wall_clock64();
+  }
   if ((int)blockIdx.x < nblk_s) {
     const int g = blockIdx.x * 256 + threadIdx.x;
     if (g < S.n) predict_point<B>(S, g);
@@ -2512,19 +2522,24 @@ void k_asm(AsmSolidArgs A, AsmFluidArgs F, RecArgs R, KwfArgs K, AsmBlocks N) {
   kwf_points<B>(K, blk % B, blk / B, N.kwf);
 }
 
-// Start of a run: each wavefield's first step and its blow-up flag cleared
-// (a kernel, not a memset: also safe where a caller captures the stream).
+// Start of a run that does not begin with k_predict (replayed graphs, initial
+// kernel wavefields): each wavefield's first step, and the clock.  The blow-up
+// flags are INT_MAX between runs (RunEnd), but for the shared buffers of
+// axh_run_noalloc, whose runs clear them here (a kernel, not a memset: also safe
+// where a caller captures the stream).
 struct StepSet {
   int *base;
   int first[kGroup];
-  int *blow[kGroup];
+  int *blow[kGroup];  // NULL: clear already
+  uint64_t *clock;
 };
 __global__ void k_step_set(StepSet A, int B) {
   const int b = threadIdx.x;
   if (b < B) {
     A.base[b] = A.first[b];
-    *A.blow[b] = INT_MAX;
+    if (A.blow[b]) *A.blow[b] = INT_MAX;
   }
+  if (b == 0) *A.clock = wall_clock64();
 }
 
 // End of a replayed graph of n steps: every wavefield n steps on.
@@ -2534,14 +2549,21 @@ __global__ void k_step_advance(int *base, int B, int n) {
 }
 
 // End of a run: the blow-up flags and the samples not yet copied out, written
-// into pinned host memory by one launch.  A copy each (from pageable memory the
-// runtime waits for the stream in every one of them) cost 12 to 20 us: a run of one
-// step of the 200 s mesh 78 -> 39 us, eight newmark2 steps of a moment tensor's four
-// wavefields on the 20 s mesh 749 -> 695 us.
+// into pinned host memory by one launch, with the device clock at the run's
+// start and end; the flags are cleared for the next run.  A copy each (from
+// pageable memory the runtime waits for the stream in every one of them) cost 12
+// to 20 us: a run of one step of the 200 s mesh 78 -> 38 us (29 us with the clock
+// instead of two events and the step base set by k_predict), eight newmark2 steps
+// of a moment tensor's four wavefields on the 20 s mesh 749 -> 695 us.
+struct RunEndHost {
+  uint64_t clock[2];
+  int blow[kGroup];
+};
 struct RunEnd {
-  int *host_blow;              // [kGroup]
+  RunEndHost *head;
+  const uint64_t *clock;
   float *host;
-  const int *blow[kGroup];
+  int *blow[kGroup];
   const float *ring[kGroup];
   // of the ring's floats `size` the n from `at` on (wrapping) go to host + off
   unsigned size[kGroup], at[kGroup], n[kGroup], off[kGroup];
@@ -2549,7 +2571,14 @@ struct RunEnd {
 __global__ __launch_bounds__(256) void k_run_end(RunEnd A) {
   const int b = blockIdx.y;
   const unsigned i = blockIdx.x * 256 + threadIdx.x;
-  if (i == 0) A.host_blow[b] = *A.blow[b];
+  if (i == 0) {
+    A.head->blow[b] = *A.blow[b];
+    *A.blow[b] = INT_MAX;
+    if (b == 0) {
+      A.head->clock[0] = *A.clock;
+      A.head->clock[1] = wall_clock64();
+    }
+  }
   if (i >= A.n[b]) return;
   unsigned x = A.at[b] + i;
   if (x >= A.size[b]) x -= A.size[b];
@@ -3352,6 +3381,7 @@ struct Fields {
   int nasm = 0;
   int *asm_pts = nullptr;
   int *step_base = nullptr;   // [kGroup] step of each wavefield (StepRef)
+  uint64_t *clock = nullptr;  // device clock at the start of the run
   // solid tiles holding a source point of the group (at most kMaxSrcTiles)
   std::vector<int> src_tiles;
 };
@@ -3431,6 +3461,7 @@ static void fields_alloc(const MeshDev &M, Fields &F, int B) {
   F.flags_s = m.alloc<uint8_t>(M.nglob_s);
   F.asm_pts = m.alloc<int>(M.nglob_s);
   F.step_base = m.zeros<int>(kGroup);
+  F.clock = m.zeros<uint64_t>(1);
   const size_t b = B;
   F.disp = m.zeros<float>(3 * (size_t)M.nglob_s * b);
   F.disp2 = m.zeros<float>(3 * (size_t)M.nglob_s * b);
@@ -3547,7 +3578,7 @@ static void member_build(const axh_ctx *ctx, const MeshDev &M, Member &W) {
     W.seis_cap = seis_staging_samples(d);
     W.seis_d = m.alloc<float>((size_t)W.seis_cap * 3 * W.nrec);
   }
-  W.blow = m.alloc<int>(1);
+  W.blow = m.upload(std::vector<int>(1, INT_MAX));
   // blow-up threshold of runtime_info: maxval(abs(disp(1,1,:,:))) >
   // 10*abs(magnitude), the real(4) maximum promoted to double
   W.blow_thr = 10.0 * std::fabs(d.magnitude);
@@ -3562,7 +3593,6 @@ constexpr size_t kRunEndFloats = (size_t)1 << 16;
 // Stream, events and per-kernel timing of the runs of a context or a batch.
 struct Runner {
   hipStream_t stream = nullptr;
-  hipEvent_t ev0 = nullptr, ev1 = nullptr;
   bool profile = false;
   bool alone = true;   // no other group's launches are queued beside these
   std::vector<hipEvent_t> kev;  // pairs
@@ -3576,25 +3606,27 @@ struct Runner {
   const int *gbase = nullptr;
   int gsteps = 0;
   uint64_t gkwf = 0;   // kernel-wavefield gather captured in the graph (0: none)
-  // pinned: the blow-up flags [kGroup] and the last samples of a run (RunEnd)
+  // pinned: the flags and clock, and the last samples of a run (RunEnd)
   unsigned char *host = nullptr;
-  int *host_blow() const { return (int *)host; }
-  float *host_samples() const { return (float *)(host + kGroup * sizeof(int)); }
+  double ticks_per_ms = 1.0;
+  RunEndHost *host_head() const { return (RunEndHost *)host; }
+  float *host_samples() const { return (float *)(host + sizeof(RunEndHost)); }
   void init() {
     if (stream) return;
-    HIPCHECK(hipHostMalloc((void **)&host, kGroup * sizeof(int) + kRunEndFloats * sizeof(float),
-                           hipHostMallocDefault));
+    int device = 0, khz = 0;
+    HIPCHECK(hipGetDevice(&device));
+    HIPCHECK(hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, device));
+    ticks_per_ms = std::max(khz, 1);
+    if (!host)
+      HIPCHECK(hipHostMalloc((void **)&host, sizeof(RunEndHost) + kRunEndFloats * sizeof(float),
+                             hipHostMallocDefault));
     HIPCHECK(hipStreamCreateWithFlags(&stream, hipStreamNonBlocking));
-    HIPCHECK(hipEventCreate(&ev0));
-    HIPCHECK(hipEventCreate(&ev1));
   }
   ~Runner() {
     // teardown: errors are not actionable here
     if (stream) (void)hipStreamSynchronize(stream);
     if (gexec) (void)hipGraphExecDestroy(gexec);
     for (auto e : kev) (void)hipEventDestroy(e);
-    if (ev0) (void)hipEventDestroy(ev0);
-    if (ev1) (void)hipEventDestroy(ev1);
     if (stream) (void)hipStreamDestroy(stream);
     if (host) (void)hipHostFree(host);
   }
@@ -3605,6 +3637,8 @@ struct Runner {
 // samples.  A context's own (run_buffers) or a fixed scratch area.
 struct RunBuffers {
   int *step_base = nullptr;
+  uint64_t *clock = nullptr;   // device clock at the start of the run
+  bool clear = true;           // the blow-up flags are INT_MAX between runs
   int *blow[kGroup] = {};
   float *ring[kGroup] = {};
   int cap[kGroup] = {};
@@ -3613,6 +3647,7 @@ struct RunBuffers {
 static RunBuffers run_buffers(Fields &F, Member *const *mb, int B) {
   RunBuffers r;
   r.step_base = F.step_base;
+  r.clock = F.clock;
   for (int b = 0; b < B; b++) {
     r.blow[b] = mb[b]->blow;
     r.ring[b] = mb[b]->seis_d;
@@ -3656,7 +3691,8 @@ struct GroupTail {
   // them as fit
   void queue_end(const Runner &R) {
     RunEnd E{};
-    E.host_blow = R.host_blow();
+    E.head = R.host_head();
+    E.clock = rb.clock;
     E.host = R.host_samples();
     size_t used = 0;
     unsigned most = 1;
@@ -3682,7 +3718,7 @@ struct GroupTail {
   // the run is complete: the staged samples to the caller
   void take_end(const Runner &R, int *blow) {
     for (int b = 0; b < B; b++) {
-      blow[b] = R.host_blow()[b];
+      blow[b] = R.host_head()->blow[b];
       if (staged[b] == 0) continue;
       const size_t row = 3 * (size_t)mb[b]->nrec;
       std::memcpy(seis[b] + (size_t)(qout[b] - q0[b]) * row, R.host_samples() + staged_at[b],
@@ -4095,14 +4131,30 @@ static void run_group(Runner &R, const MeshDev &M, Fields &F, Member *const *mb,
   Launcher L{R};
   hipStream_t st_ = R.stream;
 
-  // the run's first steps and cleared blow-up flags
+  const int S = R.graph_steps;
+  // A replay also predicts its first step and advances the step base (10 us on the
+  // 50 s mesh, 16 on 1200 x 160 elements), and saves 0.25 to 0.5 us per launch
+  // where kernels are short.  50 s mesh, replayed / direct: newmark2 in graphs of
+  // 4 steps (8 launches) 550 / 486 us, of 20 (40) 463 / 486; symplec4 anelastic of
+  // 4 (36) 1042 / 1042, of 8 (72) 1004 / 1042.  10 s mesh, of 4 (36) 2797 / 2748;
+  // kernel wavefields, of 2 (4) 1295 / 1190.  Groups queued beside others replay
+  // (the host is then what the others wait for: three groups of the 20 s mesh,
+  // 8 steps, 597 / 631).
+  const int launches = S * (M.nstages * (M.split_asm ? 3 : 2) + (M.anel || M.anel_full ? 1 : 0));
+  bool fits = S > 0 && !R.profile && nsteps >= S && (!R.alone || launches >= kReplayLaunches);
+  for (int b = 0; b < B && fits; b++)
+    fits = mb[b]->nrec <= 0 || S / std::max(mb[b]->seis_it, 1) + 1 <= RB.cap[b];
+  if (kw) fits = fits && S / kw->args.strain_it + 1 <= kw->args.cap;
+
+  // the run's first steps and its clock: set by its first k_predict, or by a
+  // launch of their own where other launches come before that one
   StepSet SS{};
   SS.base = RB.step_base;
+  SS.clock = RB.clock;
   for (int b = 0; b < B; b++) {
     SS.first[b] = start[b];
-    SS.blow[b] = RB.blow[b];
+    SS.blow[b] = RB.clear ? nullptr : RB.blow[b];
   }
-  hipLaunchKernelGGL(k_step_set, dim3(1), dim3(64), 0, st_, SS, B);
 
   SolidArgs SA{};
   SA.nel = M.nel_s; SA.nsls = M.nsls; SA.nglob = M.nglob_s; SA.nslot = (int)nslot_s;
@@ -4190,7 +4242,6 @@ static void run_group(Runner &R, const MeshDev &M, Fields &F, Member *const *mb,
     maxrec = std::max(maxrec, w.nrec);
   }
 
-  HIPCHECK(hipEventRecord(R.ev0, st_));
   T.B = B;
   T.rb = RB;
   for (int b = 0; b < B; b++) {
@@ -4199,6 +4250,15 @@ static void run_group(Runner &R, const MeshDev &M, Fields &F, Member *const *mb,
     const int si = std::max(mb[b]->seis_it, 1);
     T.q0[b] = T.qdone[b] = T.qout[b] = (start[b] - 1) / si;
   }
+  bool any0 = false;   // initial kernel wavefields
+  for (int b = 0; b < B && kw && kw->args.npt > 0; b++) any0 = any0 || start[b] == 1;
+  if (fits || any0 || !RB.clear || nsteps < 1) {
+    hipLaunchKernelGGL(k_step_set, dim3(1), dim3(64), 0, st_, SS, B);
+  } else {
+    PS.set_base = SS.base;
+    PS.set_clock = SS.clock;
+    for (int b = 0; b < B; b++) PS.first[b] = SS.first[b];
+  }
   const StepRef sref{RB.step_base, 0};
   PS.step = PF.step = FA.step = AS.step = RA.step = SA.step = sref;
   KwfArgs KA{};
@@ -4206,9 +4266,7 @@ static void run_group(Runner &R, const MeshDev &M, Fields &F, Member *const *mb,
   if (kw) {
     KA = kw->args;
     KA.step = sref;
-    bool any0 = false;
-    for (int b = 0; b < B; b++) any0 = any0 || start[b] == 1;
-    if (any0 && KA.npt > 0) {
+    if (any0) {
       // the initial fields (iter 0) of the wavefields at their first step, as
       // dump_stuff(0, ...) before the loop
       KA.step.koff = -1;
@@ -4322,20 +4380,6 @@ static void run_group(Runner &R, const MeshDev &M, Fields &F, Member *const *mb,
   };
 
   int step = 0;
-  const int S = R.graph_steps;
-  // A replay also predicts its first step and advances the step base (10 us on the
-  // 50 s mesh, 16 on 1200 x 160 elements), and saves 0.25 to 0.5 us per launch
-  // where kernels are short.  50 s mesh, replayed / direct: newmark2 in graphs of
-  // 4 steps (8 launches) 550 / 486 us, of 20 (40) 463 / 486; symplec4 anelastic of
-  // 4 (36) 1042 / 1042, of 8 (72) 1004 / 1042.  10 s mesh, of 4 (36) 2797 / 2748;
-  // kernel wavefields, of 2 (4) 1295 / 1190.  Groups queued beside others replay
-  // (the host is then what the others wait for: three groups of the 20 s mesh,
-  // 8 steps, 597 / 631).
-  const int launches = S * (M.nstages * (M.split_asm ? 3 : 2) + (M.anel || M.anel_full ? 1 : 0));
-  bool fits = S > 0 && !R.profile && nsteps >= S && (!R.alone || launches >= kReplayLaunches);
-  for (int b = 0; b < B && fits; b++)
-    fits = mb[b]->nrec <= 0 || S / std::max(mb[b]->seis_it, 1) + 1 <= RB.cap[b];
-  if (kw) fits = fits && S / kw->args.strain_it + 1 <= kw->args.cap;
   if (fits) {
     const uint64_t kgen = kw ? kw->gen : 0;
     if (!R.gexec || R.gfields != &F || R.gsteps != S || R.gbase != RB.step_base ||
@@ -4369,7 +4413,6 @@ static void run_group(Runner &R, const MeshDev &M, Fields &F, Member *const *mb,
     one_step(k, n, false, step);
   }
   HIPCHECK(hipGetLastError());
-  HIPCHECK(hipEventRecord(R.ev1, st_));
   T.queue_end(R);
 }
 
@@ -4381,8 +4424,8 @@ static double group_finish(Runner &R, GroupTail &T, int *blow) {
     if (T.staged[b] == 0) T.copy_out(b, R.stream);
   HIPCHECK(hipStreamSynchronize(R.stream));
   T.take_end(R, blow);
-  float ms = 0.0f;
-  HIPCHECK(hipEventElapsedTime(&ms, R.ev0, R.ev1));
+  const uint64_t *clock = R.host_head()->clock;
+  const double ms = (double)(int64_t)(clock[1] - clock[0]) / R.ticks_per_ms;
   if (R.profile) {
     for (size_t q = 0; q < R.kev_class.size(); q++) {
       float kms = 0.0f;
@@ -4662,9 +4705,9 @@ void batch_run(axh_batch *bt, int32_t nsteps, float *const *seis, float *const *
     for (size_t b = 0; kl && b < idx.size(); b++)
       if (kl->tail[b]) kl->tail[b]->finish(R.stream);
   }
-  // device time of the batch: first start to last end over the streams
-  // (times relative to group 0's start)
-  double first = 0.0, last = 0.0;
+  // device time of the batch: first start to last end over the streams (one
+  // clock for all of the device)
+  uint64_t first = UINT64_MAX, last = 0;
   for (size_t g = 0; g < S.groups.size(); g++) {
     int bl[kGroup];
     group_finish(*S.runs[g], tails[g], bl);
@@ -4672,13 +4715,11 @@ void batch_run(axh_batch *bt, int32_t nsteps, float *const *seis, float *const *
     for (size_t b = 0; kwf && b < idx.size(); b++)
       if (klaunch[g].tail[b]) klaunch[g].tail[b]->complete();
     for (size_t b = 0; b < idx.size(); b++) blow[idx[b]] = bl[b];
-    float t0 = 0.0f, t1 = 0.0f;
-    HIPCHECK(hipEventElapsedTime(&t0, S.runs[0]->ev0, S.runs[g]->ev0));
-    HIPCHECK(hipEventElapsedTime(&t1, S.runs[0]->ev0, S.runs[g]->ev1));
-    first = std::min(first, (double)t0);
-    last = std::max(last, (double)t1);
+    const uint64_t *clock = S.runs[g]->host_head()->clock;
+    first = std::min(first, clock[0]);
+    last = std::max(last, clock[1]);
   }
-  bt->last_run_ms = last - first;
+  bt->last_run_ms = (double)(last - first) / S.runs[0]->ticks_per_ms;
   for (axh_ctx *c : bt->members) {
     c->iter_done += nsteps;
     c->last_run_ms = bt->last_run_ms;
@@ -4698,7 +4739,7 @@ void batch_run(axh_batch *bt, int32_t nsteps, float *const *seis, float *const *
 // and finds it as the last call left it (each run sets the step base and
 // clears the flag itself); calls that overlap on one GPU race.
 constexpr size_t kScratchBytes = (size_t)AXH_NOALLOC_SCRATCH_BYTES;
-constexpr size_t kScratchHead = 256;   // step base [kGroup], blow-up flag
+constexpr size_t kScratchHead = 256;   // step base [kGroup], blow-up flag, clock
 static __device__ __align__(256) unsigned char scratch[kScratchBytes];
 constexpr int kMaxDevices = 64;
 
@@ -4735,6 +4776,8 @@ void device_run_noalloc(axh_ctx *ctx, int32_t it0, int32_t it1, float *seis) {
   Member *mb[1] = {&V.member};
   RunBuffers RB;
   RB.step_base = (int *)base;
+  RB.clock = (uint64_t *)(base + kScratchHead / 2);
+  RB.clear = false;
   RB.blow[0] = (int *)base + kGroup;
   RB.ring[0] = (float *)(base + kScratchHead);
   RB.cap[0] = (int)((kScratchBytes - kScratchHead) /

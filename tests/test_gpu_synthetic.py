@@ -9,7 +9,7 @@ launches).
 import numpy as np
 import pytest
 
-from axisem_amd.solver import Batch, Solver
+from axisem_amd.solver import Batch, BlowUp, Solver
 from axisem_amd.state import write_state
 from oracle.oracle import Oracle
 
@@ -108,3 +108,64 @@ def test_batches(scheme, anel, tmp_path):
     _check(tmp_path, "222", (5, 5), graph=3, width=2, colat=60, **o)
     _check(tmp_path, "1", (7, 6), graph=2, strain_it=3, **o)
     _check(tmp_path, "00", (4, 5), width=2, strain_it=2, **o)
+
+
+@pytest.mark.parametrize("anel", [0, 1])
+@pytest.mark.parametrize("scheme,steps", [(0, 20), (0, 21), (1, 5), (1, 6)])
+def test_replays_of_one_wavefield(scheme, steps, anel, tmp_path):
+    """Graphs of just enough launches to be replayed, and one step fewer."""
+    o = dict(scheme=scheme, anel=anel)
+    _check(tmp_path, "1", (2 * steps + 1, 2, steps), graph=steps, **o)
+    _check(tmp_path, "0", (2 * steps,), graph=steps - 1, **o)
+
+
+def test_more_samples_than_a_run_stages(tmp_path):
+    """300 receivers, 80 and 20 steps: above and below the staged samples."""
+    import perf.cases as C
+
+    case = dict(C._BASE, nth=21, nm=7, nf=3, ni=2, rec=300, src="0", steps=1)
+    s, o, d = _member(case, C._mesh(case), C, 0, 100, str(tmp_path / "s.bin"))
+    got = np.concatenate([s.run(80), s.run(20)])
+    _bits(got, o.run(1, 100, d["num_rec"], d["seis_it"]))
+    s.close()
+
+
+def test_blow_up_is_of_its_own_run(tmp_path):
+    """A run that blows up names its step; the next run starts without it."""
+    import perf.cases as C
+
+    case = dict(C._BASE, nth=21, nm=7, nf=3, ni=2, rec=15, src="0")
+    s, o, d = _member(case, C._mesh(case), C, 0, 100, str(tmp_path / "s.bin"))
+    quiet = [np.zeros_like(f) for f in s.fields()]
+    loud = [q.copy() for q in quiet]
+    loud[0][2 * loud[0].size // 3:] = 1e22
+    for _ in range(2):
+        at = s.iter + 1
+        s.set_fields(*loud)
+        with pytest.raises(BlowUp, match="time step %d$" % at):
+            s.run(3)
+        s.set_fields(*quiet)
+        s.run(4)
+        assert 0 < s.last_run_ms() < 1000
+    s.close()
+
+
+@pytest.mark.parametrize("graph", [0, 20])
+def test_no_alloc_runs(graph, tmp_path):
+    """axh_run_noalloc, whose step base, flag and ring are shared and not
+    cleared by the last run, between runs of the context's own."""
+    import perf.cases as C
+    from axisem_amd import solver as S
+
+    case = dict(C._BASE, nth=21, nm=7, nf=3, ni=2, rec=15, src="0")
+    s, o, d = _member(case, C._mesh(case), C, 0, 100, str(tmp_path / "s.bin"))
+    s.set_graph_steps(graph)
+    got = [s.run(3)]
+    for n in (21, 2, 22):
+        out = np.zeros((n, d["num_rec"], 3), np.float32)
+        S._check(S.library().axh_run_noalloc(s._h, s.iter + 1, s.iter + n, S._p(out)))
+        s.iter += n
+        got += [out, s.run(1)]
+        assert 0 < s.last_run_ms() < 1000
+    _bits(np.concatenate(got), o.run(1, s.iter, d["num_rec"], d["seis_it"]))
+    s.close()
