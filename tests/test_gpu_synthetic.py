@@ -120,10 +120,10 @@ def test_replays_of_one_wavefield(scheme, steps, anel, tmp_path):
 
 
 def test_more_samples_than_a_run_stages(tmp_path):
-    """300 receivers, 80 and 20 steps: above and below the staged samples."""
+    """1100 receivers, 80 and 20 steps: above and below the staged samples."""
     import perf.cases as C
 
-    case = dict(C._BASE, nth=21, nm=7, nf=3, ni=2, rec=300, src="0", steps=1)
+    case = dict(C._BASE, nth=21, nm=7, nf=3, ni=2, rec=1100, src="0", steps=1)
     s, o, d = _member(case, C._mesh(case), C, 0, 100, str(tmp_path / "s.bin"))
     got = np.concatenate([s.run(80), s.run(20)])
     _bits(got, o.run(1, 100, d["num_rec"], d["seis_it"]))
