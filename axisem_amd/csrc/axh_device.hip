@@ -4821,6 +4821,10 @@ static std::vector<float> fetch(const float *dsrc, size_t n, int B, int slot) {
   return out;
 }
 static void store(float *ddst, const std::vector<float> &v, int B, int slot) {
+  if (B == 1) {  // nothing of another wavefield to keep
+    HIPCHECK(hipMemcpy(ddst, v.data(), v.size() * 4, hipMemcpyHostToDevice));
+    return;
+  }
   std::vector<float> h(v.size() * B);
   HIPCHECK(hipMemcpy(h.data(), ddst, h.size() * 4, hipMemcpyDeviceToHost));
   for (size_t x = 0; x < v.size(); x++) h[x * B + slot] = v[x];
