@@ -4476,11 +4476,12 @@ void device_run_begin(axh_ctx *ctx, int32_t it0, int32_t it1, float *seis) {
 void device_run_end(axh_ctx *ctx) {
   Device &V = *ctx->dev;
   int blow = INT_MAX;
-  ctx->last_run_ms = group_finish(V.run, V.pending, &blow);
+  // (the snapshots first: an earlier piece is moved while the last steps run)
   if (V.pending_has_kwf) {
     V.pending_has_kwf = false;
     V.pending_kwf.complete();
   }
+  ctx->last_run_ms = group_finish(V.run, V.pending, &blow);
   ctx->iter_done = V.pending_it1;
   if (blow != INT_MAX)
     fail(AXH_ERR_BLOWUP, "displacements blew up at time step " + std::to_string(blow));
@@ -4495,7 +4496,11 @@ void device_run(axh_ctx *ctx, int32_t it0, int32_t it1, float *seis) {
 // kernel-wavefield runs (axh_run_kwf)
 // ---------------------------------------------------------------------------
 constexpr size_t kKwfRingBytes = AXH_KWF_RING_BYTES;  // snapshot ring on the device
-constexpr size_t kKwfStageBytes = (size_t)16 << 20;   // one pinned staging half
+// One pinned staging half: small enough that short runs and small grids move their
+// first snapshots while later steps run (20 s mesh, 26 steps with 3 snapshots of 3
+// MB: halves of 16 MiB 1179, of 4 MiB 1124, of 2 MiB 1150 us; 260 steps with 21
+// 10.1, 9.5, 9.6 ms; 50 s mesh, 30 of 0.8 MB in 60 steps 2239, 1732, 1785 us).
+constexpr size_t kKwfStageBytes = (size_t)4 << 20;
 
 // The point tables of k_kwf from the context's grid, in point order: the
 // solid points' global ids (-1 in a source element when src_mask), the fluid
@@ -4553,7 +4558,7 @@ static void kwf_build(axh_ctx *ctx, Device &V) {
   const size_t snap = (size_t)K->ncomp * std::max(npt, 1);
   const size_t snap_b = snap * sizeof(float);
   const int total = d.niter / K->strain_it + 1;
-  // staging halves of up to 16 MiB (at least one snapshot); the ring holds two halves and the
+  // staging halves of up to 4 MiB (at least one snapshot); the ring holds two halves and the
   // snapshots of one replayed graph (at least 2 slots: a run from step 1
   // takes the initial snapshot and the first), at most 1 GiB
   if (ctx->kwf_ring > 0) {
@@ -4711,10 +4716,10 @@ void batch_run(axh_batch *bt, int32_t nsteps, float *const *seis, float *const *
   uint64_t first = UINT64_MAX, last = 0;
   for (size_t g = 0; g < S.groups.size(); g++) {
     int bl[kGroup];
-    group_finish(*S.runs[g], tails[g], bl);
     const std::vector<int> &idx = S.index[g];
     for (size_t b = 0; kwf && b < idx.size(); b++)
       if (klaunch[g].tail[b]) klaunch[g].tail[b]->complete();
+    group_finish(*S.runs[g], tails[g], bl);
     for (size_t b = 0; b < idx.size(); b++) blow[idx[b]] = bl[b];
     const uint64_t *clock = S.runs[g]->host_head()->clock;
     first = std::min(first, clock[0]);

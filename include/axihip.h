@@ -484,7 +484,7 @@ int axh_kwf_get_grid(const axh_ctx *ctx, int32_t *mapping_ijel_ikwf, int32_t *kw
  * SOLVER/wavefields_io.f90:1123-1135), 0 keeps it ('none').  ring_snapshots
  * sets the device ring the snapshots are gathered in (at least 2; 0: chosen
  * by the library, at most AXH_KWF_RING_BYTES); they are copied out half a
- * ring (at most 16 MiB, at least one snapshot) at a time.  Any time. */
+ * ring (at most 4 MiB, at least one snapshot) at a time.  Any time. */
 #define AXH_KWF_RING_BYTES ((size_t)1 << 30)
 int axh_set_kwf(axh_ctx *ctx, int32_t strain_it, int32_t src_mask, int32_t ring_snapshots);
 
