@@ -1707,7 +1707,7 @@ __global__ __launch_bounds__(256) void k_memvar(SolidArgs A, RecArgs R) {
 // instead of 6 n_sls.
 // ---------------------------------------------------------------------------
 struct AnelFullArgs {
-  int nel, nsls, nglob;
+  int nel, nsls, nglob, ntile;
   const float *G;         // G0 | G1 | G1T | G2 | G2T
   const float *terms;     // [tile][kAfTerms][256]
   const int *einfo, *gid;
@@ -1729,12 +1729,17 @@ struct AnelFullArgs {
 // elements, dipole: 42.9 -> 37 us (6.1 TB/s); whole steps: 2 monopoles 883 -> 824
 // us, monopole newmark2 761 -> 718 us, group of 4 dipoles 1757 -> 1739 us.
 template <int SRC, int B, int MS>
-__global__ __launch_bounds__(256) void k_anel_full(AnelFullArgs A) {
+__global__ __launch_bounds__(256) void k_anel_full(AnelFullArgs A, RecArgs R) {
   __shared__ float sG[105];
   __shared__ float sA[5][256 * B];  // the strain's fields
   // ts_fac_t(q) a_j, ts_fac_tm1(q) a_j per element (mu, then kappa)
   __shared__ double sCf[kElemPerTile][MS][4];
   const int t = threadIdx.x, tile = blockIdx.x;
+  if (tile >= A.ntile) {  // receiver samples, as in k_memvar (block-uniform)
+    const int q = tile - A.ntile;
+    rec_sample<B>(R, (q / B) * 256 + t, q % B);
+    return;
+  }
   const int le = t / 25, k = t - 25 * le;
   const int i = k % 5, j = k / 5;
   const int e = tile * kElemPerTile + le;
@@ -4057,19 +4062,21 @@ static void dispatch_solid(const MeshDev &M, hipStream_t s, const SolidArgs &A,
 }
 
 template <int B, int MS>
-static void dispatch_anel_full_ms(const MeshDev &M, hipStream_t s, const AnelFullArgs &A) {
-  const dim3 grid(M.ntile_s), blk(256);
+static void dispatch_anel_full_ms(const MeshDev &M, hipStream_t s, const AnelFullArgs &A,
+                                  const RecArgs &R, int nrec_blk) {
+  const dim3 grid(M.ntile_s + nrec_blk), blk(256);
   if (M.src == AXH_MONOPOLE)
-    hipLaunchKernelGGL((k_anel_full<AXH_MONOPOLE, B, MS>), grid, blk, 0, s, A);
+    hipLaunchKernelGGL((k_anel_full<AXH_MONOPOLE, B, MS>), grid, blk, 0, s, A, R);
   else if (M.src == AXH_DIPOLE)
-    hipLaunchKernelGGL((k_anel_full<AXH_DIPOLE, B, MS>), grid, blk, 0, s, A);
+    hipLaunchKernelGGL((k_anel_full<AXH_DIPOLE, B, MS>), grid, blk, 0, s, A, R);
   else
-    hipLaunchKernelGGL((k_anel_full<AXH_QUADPOLE, B, MS>), grid, blk, 0, s, A);
+    hipLaunchKernelGGL((k_anel_full<AXH_QUADPOLE, B, MS>), grid, blk, 0, s, A, R);
 }
 template <int B>
-static void dispatch_anel_full(const MeshDev &M, hipStream_t s, const AnelFullArgs &A) {
-  if (M.nsls <= 5) dispatch_anel_full_ms<B, 5>(M, s, A);
-  else dispatch_anel_full_ms<B, kMaxSls>(M, s, A);
+static void dispatch_anel_full(const MeshDev &M, hipStream_t s, const AnelFullArgs &A,
+                               const RecArgs &R, int nrec_blk) {
+  if (M.nsls <= 5) dispatch_anel_full_ms<B, 5>(M, s, A, R, nrec_blk);
+  else dispatch_anel_full_ms<B, kMaxSls>(M, s, A, R, nrec_blk);
 }
 
 // the SLS capacity of the kernel: 5 (the reference's default number of
@@ -4178,7 +4185,7 @@ static void run_group(Runner &R, const MeshDev &M, Fields &F, Member *const *mb,
   SA.blow = RB.blow[0]; SA.thr = mb[0]->blow_thr;
   AnelFullArgs AN{};
   if (M.anel_full) {
-    AN.nel = M.nel_s; AN.nsls = M.nsls; AN.nglob = M.nglob_s;
+    AN.nel = M.nel_s; AN.ntile = M.ntile_s; AN.nsls = M.nsls; AN.nglob = M.nglob_s;
     AN.G = M.G; AN.terms = M.af_terms; AN.einfo = M.einfo_s;
     AN.gid = M.gid_s; AN.aj_mu = M.aj_mu; AN.aj_k = M.aj_k;
     for (int s = 0; s < kMaxSls; s++) {
@@ -4357,14 +4364,14 @@ static void run_group(Runner &R, const MeshDev &M, Fields &F, Member *const *mb,
                            st_, AS, AF, RA, KA, N);
       });
     }
-    if (M.anel_full) L(KC_MEMVAR, [&] { dispatch_anel_full<B>(M, st_, AN); });
+    // a symplectic step's receiver samples ride along as extra blocks of the
+    // memory-variable update (newmark2's are in the assembly); at all 25 points, 24 480
+    // elements, dipole, 6 steps: 1012 -> 995 us
+    const int nrb = any && !newmark ? nblk(maxrec) * B : 0;
+    if (M.anel_full) L(KC_MEMVAR, [&] { dispatch_anel_full<B>(M, st_, AN, RA, nrb); });
     if (newmark) return;
-    if (M.anel) {
-      // the receiver samples ride along as extra blocks of the update
-      const int nrb = any ? nblk(maxrec) * B : 0;
-      L(KC_MEMVAR, [&] { dispatch_memvar<B>(M, st_, SA, RA, nrb); });
-      any = false;
-    }
+    if (M.anel) L(KC_MEMVAR, [&] { dispatch_memvar<B>(M, st_, SA, RA, nrb); });
+    if (M.anel || M.anel_full) any = false;
     if (any)
       L(KC_REC, [&] {
         hipLaunchKernelGGL(k_receivers<B>, dim3(nblk(maxrec), B), dim3(256), 0, st_, RA);
