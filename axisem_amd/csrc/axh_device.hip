@@ -3600,13 +3600,17 @@ constexpr size_t kRunEndFloats = (size_t)1 << 18;
 struct Runner {
   hipStream_t stream = nullptr;
   bool profile = false;
-  bool alone = true;   // no other group's launches are queued beside these
+  // a run of one group that its caller waits for; a queued run, and a group among
+  // others, replays graphs of any length: the host is then what others wait for (three
+  // groups of the 20 s mesh, 8 steps, 597 us replayed, 631 direct)
+  bool alone = true;
   std::vector<hipEvent_t> kev;  // pairs
   std::vector<int> kev_class;
   double kms[KC_N] = {0};
   long kcount[KC_N] = {0};
   // replayed graph of graph_steps steps of one group (0: launch directly)
   int graph_steps = 0;
+  int replays = 0;     // graphs replayed by the last run
   hipGraphExec_t gexec = nullptr;
   const void *gfields = nullptr;
   const int *gbase = nullptr;
@@ -4123,7 +4127,25 @@ struct KwfLaunch {
   KwfTail *tail[kGroup] = {};
 };
 constexpr int kKwfBlocks = 1024;   // grid of k_kwf (grid-stride over the points)
-constexpr int kReplayLaunches = 40;  // fewest launches of a graph that is replayed
+
+// Fewest launches of a graph that a run of one group replays; a shorter one's steps
+// are launched directly.  A replay also predicts its first step, advances the step
+// base and waits for the graph before it (8 us on the 200 s mesh, 16 on 108 000
+// elements), and saves up to 1.2 us per launch where kernels are shorter than their
+// launches, nothing where they are longer.  Replayed / direct, us per graph:
+//   972 elements (200 s), newmark2, 8 launches: 64.5 / 62.5, 16: 102.6 / 103.5, 32: 174.5
+//   / 188.8; symplec4 anelastic, 18: 129.2 / 135.9, 36: 228.3 / 247.3; 4 wavefields,
+//   newmark2, 16: 144.0 / 140.9, 32: 243.5 / 248.5
+//   6 072 (50 s), newmark2, 8: 73.3 / 72.7, 16: 114.7 / 120.3, 32: 199.3 / 215.2;
+//   symplec4 anelastic, 18: 152.3 / 151.6, 36: 272.0 / 273.1; 2 wavefields, newmark2, 16:
+//   136.5 / 135.2, 40: 280.3 / 287.3; 4 wavefields, 16: 184.9 / 177.0, 64: 597.6 / 596.1
+//   12 000, newmark2, 16: 142.3 / 140.4, 32: 253.3 / 252.1, 64: 475.8 / 488.6
+//   108 000, newmark2, 16: 488.1 / 478.7, 64: 1852 / 1833
+// From 40 launches on every mesh replays, as the caller asked: it costs at most 3 % and
+// frees the host.
+static int replay_launches(long elements, int wavefields) {
+  return elements * wavefields > 8000 ? 40 : 16;
+}
 
 template <int B>
 static void run_group(Runner &R, const MeshDev &M, Fields &F, Member *const *mb,
@@ -4138,21 +4160,6 @@ static void run_group(Runner &R, const MeshDev &M, Fields &F, Member *const *mb,
   const size_t nslot_s = (size_t)M.ntile_s * kTile;
   Launcher L{R};
   hipStream_t st_ = R.stream;
-
-  const int S = R.graph_steps;
-  // A replay also predicts its first step and advances the step base (10 us on the
-  // 50 s mesh, 16 on 1200 x 160 elements), and saves 0.25 to 0.5 us per launch
-  // where kernels are short.  50 s mesh, replayed / direct: newmark2 in graphs of
-  // 4 steps (8 launches) 550 / 486 us, of 20 (40) 463 / 486; symplec4 anelastic of
-  // 4 (36) 1042 / 1042, of 8 (72) 1004 / 1042.  10 s mesh, of 4 (36) 2797 / 2748;
-  // kernel wavefields, of 2 (4) 1295 / 1190.  Groups queued beside others replay
-  // (the host is then what the others wait for: three groups of the 20 s mesh,
-  // 8 steps, 597 / 631).
-  const int launches = S * (M.nstages * (M.split_asm ? 3 : 2) + (M.anel || M.anel_full ? 1 : 0));
-  bool fits = S > 0 && !R.profile && nsteps >= S && (!R.alone || launches >= kReplayLaunches);
-  for (int b = 0; b < B && fits; b++)
-    fits = mb[b]->nrec <= 0 || S / std::max(mb[b]->seis_it, 1) + 1 <= RB.cap[b];
-  if (kw) fits = fits && S / kw->args.strain_it + 1 <= kw->args.cap;
 
   // the run's first steps and its clock: set by its first k_predict, or by a
   // launch of their own where other launches come before that one
@@ -4249,6 +4256,19 @@ static void run_group(Runner &R, const MeshDev &M, Fields &F, Member *const *mb,
     RA.seis_it[b] = std::max(w.seis_it, 1); RA.cap[b] = RB.cap[b];
     maxrec = std::max(maxrec, w.nrec);
   }
+
+  // the launches one_step queues for a step of a graph
+  const int S = R.graph_steps;
+  const int per_step = M.nstages * (M.split_asm ? 3 : 2) +
+                       (M.anel_full || (M.anel && !newmark) ? 1 : 0) +
+                       (!newmark && !M.anel && !M.anel_full && maxrec > 0 ? 1 : 0) +
+                       (!newmark && kw && kw->args.npt > 0 ? 1 : 0);
+  bool fits = S > 0 && !R.profile && nsteps >= S &&
+              (!R.alone || S * per_step >= replay_launches((long)M.nel_s + M.nel_f, B));
+  for (int b = 0; b < B && fits; b++)
+    fits = mb[b]->nrec <= 0 || S / std::max(mb[b]->seis_it, 1) + 1 <= RB.cap[b];
+  if (kw) fits = fits && S / kw->args.strain_it + 1 <= kw->args.cap;
+  R.replays = 0;
 
   T.B = B;
   T.rb = RB;
@@ -4413,6 +4433,7 @@ static void run_group(Runner &R, const MeshDev &M, Fields &F, Member *const *mb,
     for (; step + S <= nsteps; step += S) {
       reserve(step, S);
       HIPCHECK(hipGraphLaunch(R.gexec, st_));
+      R.replays++;
     }
   }
   // the rest, launched directly (koff counts from the current step base)
@@ -4463,11 +4484,13 @@ static void run_any(Runner &R, const MeshDev &M, Fields &F, Member *const *mb,
 
 // Queues steps it0..it1 of a context on its stream; device_run_end
 // completes them.  Between the two the host is free (e.g. to write the
-// previous run's samples) and seis must stay untouched.
-void device_run_begin(axh_ctx *ctx, int32_t it0, int32_t it1, float *seis) {
+// previous run's samples) and seis must stay untouched.  waits: the caller goes
+// straight on to device_run_end.
+void device_run_begin(axh_ctx *ctx, int32_t it0, int32_t it1, float *seis, bool waits) {
   Device &V = *ctx->dev;
   if (V.live) fail(AXH_ERR_STATE, "the context is stepped by a batch");
   V.run.init();
+  V.run.alone = waits;
   V.run.profile = ctx->profile;
   V.run.graph_steps = ctx->graph_steps;
   Member *mb[1] = {&V.member};
@@ -4489,13 +4512,14 @@ void device_run_end(axh_ctx *ctx) {
     V.pending_kwf.complete();
   }
   ctx->last_run_ms = group_finish(V.run, V.pending, &blow);
+  ctx->last_run_replays = V.run.replays;
   ctx->iter_done = V.pending_it1;
   if (blow != INT_MAX)
     fail(AXH_ERR_BLOWUP, "displacements blew up at time step " + std::to_string(blow));
 }
 
 void device_run(axh_ctx *ctx, int32_t it0, int32_t it1, float *seis) {
-  device_run_begin(ctx, it0, it1, seis);
+  device_run_begin(ctx, it0, it1, seis, true);
   device_run_end(ctx);
 }
 
@@ -4646,7 +4670,8 @@ static void kwf_group(KwfDev *const *K, int B, const MeshDev &M, const Fields &F
 // device_run_end completes them.  The snapshots are copied out through the
 // pinned staging halves while the following steps run (KwfTail); between the
 // two calls the host is free, and seis and kwf must stay untouched.
-void device_run_kwf_begin(axh_ctx *ctx, int32_t it0, int32_t it1, float *seis, float *kwf) {
+void device_run_kwf_begin(axh_ctx *ctx, int32_t it0, int32_t it1, float *seis, float *kwf,
+                          bool waits) {
   Device &V = *ctx->dev;
   if (V.live) fail(AXH_ERR_STATE, "the context is stepped by a batch");
   KwfDev *K[1] = {&kwf_of(ctx)};
@@ -4656,6 +4681,7 @@ void device_run_kwf_begin(axh_ctx *ctx, int32_t it0, int32_t it1, float *seis, f
   kwf_group(K, 1, *V.mesh, V.own, start, kout, kl, &V.pending_kwf);
   V.pending_has_kwf = kl.tail[0] != nullptr;
   V.run.init();
+  V.run.alone = waits;
   V.run.profile = ctx->profile;
   V.run.graph_steps = ctx->graph_steps;
   Member *mb[1] = {&V.member};
@@ -4669,7 +4695,7 @@ void device_run_kwf_begin(axh_ctx *ctx, int32_t it0, int32_t it1, float *seis, f
 }
 
 void device_run_kwf(axh_ctx *ctx, int32_t it0, int32_t it1, float *seis, float *kwf) {
-  device_run_kwf_begin(ctx, it0, it1, seis, kwf);
+  device_run_kwf_begin(ctx, it0, it1, seis, kwf, true);
   device_run_end(ctx);
 }
 
@@ -4727,7 +4753,10 @@ void batch_run(axh_batch *bt, int32_t nsteps, float *const *seis, float *const *
     for (size_t b = 0; kwf && b < idx.size(); b++)
       if (klaunch[g].tail[b]) klaunch[g].tail[b]->complete();
     group_finish(*S.runs[g], tails[g], bl);
-    for (size_t b = 0; b < idx.size(); b++) blow[idx[b]] = bl[b];
+    for (size_t b = 0; b < idx.size(); b++) {
+      blow[idx[b]] = bl[b];
+      bt->members[idx[b]]->last_run_replays = S.runs[g]->replays;
+    }
     const uint64_t *clock = S.runs[g]->host_head()->clock;
     first = std::min(first, clock[0]);
     last = std::max(last, clock[1]);
@@ -4797,6 +4826,7 @@ void device_run_noalloc(axh_ctx *ctx, int32_t it0, int32_t it1, float *seis) {
                     (3 * sizeof(float) * (size_t)std::max(V.member.nrec, 1)));
   // per-kernel profiling creates events: off for this entry point
   V.run.profile = false;
+  V.run.alone = true;
   V.run.graph_steps = ctx->graph_steps;
   const axh_ctx *cx[1] = {ctx};
   float *out[1] = {seis};
@@ -4805,6 +4835,7 @@ void device_run_noalloc(axh_ctx *ctx, int32_t it0, int32_t it1, float *seis) {
   GroupTail T;
   run_any(V.run, *V.mesh, V.own, mb, cx, start, it1 - it0 + 1, out, RB, T);
   ctx->last_run_ms = group_finish(V.run, T, &blow);
+  ctx->last_run_replays = V.run.replays;
   ctx->iter_done = it1;
   if (blow != INT_MAX)
     fail(AXH_ERR_BLOWUP, "displacements blew up at time step " + std::to_string(blow));

@@ -450,6 +450,14 @@ int axh_last_run_ms(const axh_ctx *ctx, double *total_ms) {
   });
 }
 
+int axh_last_run_replays(const axh_ctx *ctx, int32_t *replays) {
+  return guarded([&] {
+    check_ctx(ctx);
+    if (!replays) fail(AXH_ERR_ARG, "null pointer");
+    *replays = ctx->last_run_replays;
+  });
+}
+
 int axh_check_inputs(axh_ctx *ctx) {
   return guarded([&] {
     check_ctx(ctx);

@@ -80,6 +80,7 @@ struct axh_ctx {
   std::unique_ptr<axh::Device, axh::DeviceDeleter> dev;
   int32_t iter_done = 0;  // last completed step
   double last_run_ms = 0.0;
+  int last_run_replays = 0;  // graphs replayed by the last run
   bool profile = false;
   int graph_steps = 0;    // steps per replayed graph (0: direct launches)
   bool running = false;   // between axh_run_begin and axh_run_end
@@ -127,11 +128,12 @@ extern const char *const kFluidGradNames[5];
 void device_build(axh_ctx *ctx);
 void device_destroy(Device *d);
 void device_run(axh_ctx *ctx, int32_t it0, int32_t it1, float *seis);
-void device_run_begin(axh_ctx *ctx, int32_t it0, int32_t it1, float *seis);
+void device_run_begin(axh_ctx *ctx, int32_t it0, int32_t it1, float *seis, bool waits = false);
 void device_run_end(axh_ctx *ctx);
 void device_run_noalloc(axh_ctx *ctx, int32_t it0, int32_t it1, float *seis);
 void device_run_kwf(axh_ctx *ctx, int32_t it0, int32_t it1, float *seis, float *kwf);
-void device_run_kwf_begin(axh_ctx *ctx, int32_t it0, int32_t it1, float *seis, float *kwf);
+void device_run_kwf_begin(axh_ctx *ctx, int32_t it0, int32_t it1, float *seis, float *kwf,
+                          bool waits = false);
 void convolve_traces(int nt, int ntraces, const float *seis, int nj, const float *stf,
                      double dt, double scale, float *out);
 int noalloc_max_receivers();

@@ -115,6 +115,7 @@ def library(fused: bool = False):
         L.axh_download_fields.argtypes = [P, P, P, P, P, P]
         L.axh_upload_fields.argtypes = [P, P, P, P, P, P]
         L.axh_last_run_ms.argtypes = [P, C.POINTER(C.c_double)]
+        L.axh_last_run_replays.argtypes = [P, C.POINTER(C.c_int32)]
         L.axh_device_bytes.argtypes = [P, C.POINTER(C.c_size_t)]
         L.axh_kernel_stats.argtypes = [P, C.c_int, C.POINTER(C.c_double), C.POINTER(C.c_int64)]
         L.axh_kernel_name.restype = C.c_char_p
@@ -427,6 +428,12 @@ class Solver:
         self._ok(self._L.axh_last_run_ms(self._h, C.byref(v)))
         return v.value
 
+    def last_run_replays(self) -> int:
+        """Graphs the last run replayed (0: launched directly)."""
+        v = C.c_int32()
+        self._ok(self._L.axh_last_run_replays(self._h, C.byref(v)))
+        return v.value
+
     def device_bytes(self) -> int:
         v = C.c_size_t()
         self._ok(self._L.axh_device_bytes(self._h, C.byref(v)))
@@ -437,7 +444,9 @@ class Solver:
 
     def set_graph_steps(self, steps: int):
         """Replay a captured HIP graph of `steps` time steps (0: launch every
-        kernel directly); results are identical either way."""
+        kernel directly); results are identical either way.  Runs whose graph
+        would hold few launches are launched directly (axh_set_graph_steps);
+        last_run_replays() tells."""
         self._ok(self._L.axh_set_graph_steps(self._h, steps))
 
     def kernel_stats(self) -> dict:
@@ -572,6 +581,10 @@ class Batch:
         v = C.c_double()
         self._ok(self._L.axh_batch_last_run_ms(self._h, C.byref(v)))
         return v.value
+
+    def last_run_replays(self) -> int:
+        """Graphs the last run replayed, of the group with the most."""
+        return max(s.last_run_replays() for s in self.solvers)
 
     def set_profiling(self, on: bool):
         self._ok(self._L.axh_batch_set_profiling(self._h, 1 if on else 0))

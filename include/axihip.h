@@ -271,8 +271,8 @@ int axh_download_fields(axh_ctx *ctx, float *disp, float *velo, float *chi,
 int axh_upload_fields(axh_ctx *ctx, const float *disp, const float *velo,
                       const float *chi, const float *dchi, const float *ddchi);
 
-/* Time spent in the last axh_run on the device, from HIP events on the
- * library stream [ms]. */
+/* Time spent in the last axh_run on the device, from the device clock read by
+ * the run's first and last kernel [ms]. */
 int axh_last_run_ms(const axh_ctx *ctx, double *total_ms);
 
 /* Per-kernel timing.  When on, every kernel launch of axh_run is bracketed by
@@ -285,14 +285,23 @@ int axh_kernel_stats(const axh_ctx *ctx, int kclass, double *total_ms,
 
 /* Launch mode of axh_run: steps = 0 launches every kernel directly (the
  * default); steps = S > 0 captures S time steps of the context once into a
- * HIP graph and replays it for every S steps of a run (the rest of a run,
- * runs with per-kernel profiling on, and runs that are faster so -- one group
- * and a graph of fewer than 40 launches -- launch directly).  Each kernel reads
+ * HIP graph and replays it for every S steps of a run (the rest of a run and
+ * runs with per-kernel profiling on launch directly).  Each kernel reads
  * its time step from device memory, so the replays need no host work per
  * step; results are bit-identical either way.  Small meshes, whose steps are
- * bound by launch latency, gain.  The reference has no counterpart (its time
+ * bound by launch latency, gain.  A run that its caller waits for (axh_run,
+ * axh_run_kwf, axh_run_noalloc, a batch of one group) and whose graph would hold
+ * few launches is launched directly, which is faster: fewer than 16 launches for up
+ * to 8000 elements (times the wavefields of the group), fewer than 40 beyond.
+ * Queued runs and groups that run beside others always replay.  A newmark2 step is
+ * 2 launches, a symplectic one 2 per stage and 1 for attenuation (with absorbing
+ * boundaries 3 for 2).  The reference has no counterpart (its time
  * loop is a host loop, SOLVER/time_evol_wave.F90:353-500). */
 int axh_set_graph_steps(axh_ctx *ctx, int32_t steps);
+
+/* Graphs replayed by the last run of the context (for a member of a batch: by
+ * its group's last run); 0 when all of its steps were launched directly. */
+int axh_last_run_replays(const axh_ctx *ctx, int32_t *replays);
 
 /* Device memory held by the context [bytes] (0 before the first run). */
 int axh_device_bytes(axh_ctx *ctx, size_t *bytes);
