@@ -47,6 +47,7 @@
 #include <vector>
 
 #include "axh_internal.h"
+#include "axh_pool.h"
 
 #ifdef AXH_FUSED_MULTIPLY_ADD
 #pragma clang fp contract(fast)
@@ -3460,40 +3461,55 @@ static void fields_set_sources(const MeshDev &M, Fields &F,
     HIPCHECK(hipMemcpy(F.asm_pts, pts.data(), pts.size() * sizeof(int), hipMemcpyHostToDevice));
 }
 
-static void fields_alloc(const MeshDev &M, Fields &F, int B) {
-  F.B = B;
-  DevAlloc &m = F.mem;
-  F.flags_s = m.alloc<uint8_t>(M.nglob_s);
-  F.asm_pts = m.alloc<int>(M.nglob_s);
-  F.step_base = m.zeros<int>(kGroup);
-  F.clock = m.zeros<uint64_t>(1);
-  const size_t b = B;
-  F.disp = m.zeros<float>(3 * (size_t)M.nglob_s * b);
-  F.disp2 = m.zeros<float>(3 * (size_t)M.nglob_s * b);
-  F.velo = m.zeros<float>(3 * (size_t)M.nglob_s * b);
-  F.acc0 = m.zeros<float>(3 * (size_t)M.nglob_s * b);
-  F.force_s = m.zeros<float>(3 * (size_t)M.ntile_s * kTile * b);
-  F.axb_val = m.zeros<float>(3 * (size_t)std::max(M.naxb, 1) * b);
+// Sets the arrays of F in a block that starts at base (NULL: only counts) and returns the
+// bytes of the block.
+static size_t fields_layout(const MeshDev &M, Fields &F, char *base) {
+  size_t at = 0;
+  auto part = [&](auto *&p, size_t n) {
+    using T = std::remove_reference_t<decltype(*p)>;
+    if (base) p = (T *)(base + at);
+    at += (std::max<size_t>(n, 1) * sizeof(T) + 255) / 256 * 256;
+  };
+  const size_t b = F.B;
+  part(F.flags_s, M.nglob_s);
+  part(F.asm_pts, M.nglob_s);
+  part(F.step_base, kGroup);
+  part(F.clock, 1);
+  part(F.disp, 3 * (size_t)M.nglob_s * b);
+  part(F.disp2, 3 * (size_t)M.nglob_s * b);
+  part(F.velo, 3 * (size_t)M.nglob_s * b);
+  part(F.acc0, 3 * (size_t)M.nglob_s * b);
+  part(F.force_s, 3 * (size_t)M.ntile_s * kTile * b);
+  part(F.axb_val, 3 * (size_t)std::max(M.naxb, 1) * b);
   if (M.nel_f > 0) {
-    F.chi = m.zeros<float>((size_t)M.nglob_f * b);
-    F.chi2 = m.zeros<float>((size_t)M.nglob_f * b);
-    F.dchi = m.zeros<float>((size_t)M.nglob_f * b);
-    F.ddchi = m.zeros<float>((size_t)M.nglob_f * b);
-    F.force_f = m.zeros<float>((size_t)M.ntile_f * kTile * b);
+    part(F.chi, (size_t)M.nglob_f * b);
+    part(F.chi2, (size_t)M.nglob_f * b);
+    part(F.dchi, (size_t)M.nglob_f * b);
+    part(F.ddchi, (size_t)M.nglob_f * b);
+    part(F.force_f, (size_t)M.ntile_f * kTile * b);
   }
   if (M.anel) {
-    F.memvar = m.zeros<float>((size_t)M.nel_s * 24 * M.nsls * b);
-    F.rsum = m.zeros<float>((size_t)M.nel_s * 24 * b);
-    F.trm1 = m.zeros<float>((size_t)M.nel_s * 4 * b);
-    F.devm1 = m.zeros<float>((size_t)M.nel_s * 24 * b);
+    part(F.memvar, (size_t)M.nel_s * 24 * M.nsls * b);
+    part(F.rsum, (size_t)M.nel_s * 24 * b);
+    part(F.trm1, (size_t)M.nel_s * 4 * b);
+    part(F.devm1, (size_t)M.nel_s * 24 * b);
   }
   if (M.anel_full) {
     const size_t ns = (size_t)M.ntile_s * kTile;
-    F.memvar = m.zeros<float>(ns * 6 * M.nsls * b);
-    F.rsum = m.zeros<float>(ns * 6 * b);
-    F.trm1 = m.zeros<float>(ns * b);
-    F.devm1 = m.zeros<float>(ns * 6 * b);
+    part(F.memvar, ns * 6 * M.nsls * b);
+    part(F.rsum, ns * 6 * b);
+    part(F.trm1, ns * b);
+    part(F.devm1, ns * 6 * b);
   }
+  return at;
+}
+
+// All of a group's arrays in one allocation: the first run of a batch makes them, and an
+// allocation of more than 2 MB takes 30 to 600 us (three groups of the 20 s mesh: 2.2 ms
+// in 39 of them; the batch's first run 5.9 -> 4.7 ms).
+static void fields_alloc(const MeshDev &M, Fields &F, int B) {
+  F.B = B;
+  fields_layout(M, F, F.mem.zeros<char>(fields_layout(M, F, nullptr)));
 }
 
 // Copy wavefield src_b of S into wavefield dst_b of D (same mesh), through
@@ -3596,6 +3612,21 @@ static void member_build(const axh_ctx *ctx, const MeshDev &M, Member &W) {
 // of it as they need)
 constexpr size_t kRunEndFloats = (size_t)1 << 18;
 
+// The pinned blocks of the runners.  Pinned by every first run they cost it 50 us, and
+// the three groups of a moment tensor 0.17 to 0.5 ms (first run of a new context, one step
+// of the 200 s mesh: 200 -> 112 us).
+static BlockPool &run_end_blocks() {
+  static BlockPool *const pool = new BlockPool(
+      [] {
+        void *p = nullptr;
+        HIPCHECK(hipHostMalloc(&p, sizeof(RunEndHost) + kRunEndFloats * sizeof(float),
+                               hipHostMallocPortable));
+        return p;
+      },
+      [](void *p) { (void)hipHostFree(p); }, 4);
+  return *pool;
+}
+
 // Stream, events and per-kernel timing of the runs of a context or a batch.
 struct Runner {
   hipStream_t stream = nullptr;
@@ -3627,9 +3658,7 @@ struct Runner {
     HIPCHECK(hipGetDevice(&device));
     HIPCHECK(hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, device));
     ticks_per_ms = std::max(khz, 1);
-    if (!host)
-      HIPCHECK(hipHostMalloc((void **)&host, sizeof(RunEndHost) + kRunEndFloats * sizeof(float),
-                             hipHostMallocDefault));
+    if (!host) host = (unsigned char *)run_end_blocks().take();
     HIPCHECK(hipStreamCreateWithFlags(&stream, hipStreamNonBlocking));
   }
   ~Runner() {
@@ -3638,7 +3667,7 @@ struct Runner {
     if (gexec) (void)hipGraphExecDestroy(gexec);
     for (auto e : kev) (void)hipEventDestroy(e);
     if (stream) (void)hipStreamDestroy(stream);
-    if (host) (void)hipHostFree(host);
+    if (host) run_end_blocks().give(host);
   }
 };
 
