@@ -2018,7 +2018,7 @@ __global__ __launch_bounds__(256) void k_predict(PredArgs S, PredArgs F, int nbl
 // assembly + mass + update, per global point
 // ---------------------------------------------------------------------------
 struct AsmSolidArgs {
-  int n, src, newmark, nslot, comps, mask0, mask1;
+  int n, src, nslot, comps, mask0, mask1;
   int npts;              // points assembled here (the others are kFlagDirect)
   int ncontig;           // pts[ip] == ip for ip < ncontig (not read there)
   const int *pts;
@@ -2038,7 +2038,7 @@ struct AsmSolidArgs {
   int nstages, stage;
   // symplectic: the drift of the next stage (or the final drift) right after
   // the kick, u = u + v*cd_next, masked when drift_mask is set
-  int drift, drift_mask, naxb;
+  int drift_mask, naxb;
   double cd_next;
   float *disp;           // [3][n][B]
   // the next step's predictor (first drift) with the axis mask and the
@@ -2065,7 +2065,7 @@ struct AsmSolidArgs {
 };
 
 struct AsmFluidArgs {
-  int n, newmark, mask_axis;
+  int n, mask_axis;
   const int4 *copies;        // point_copies, none where the force is masked
   const int *gstart, *gslot;
   const uint8_t *flags;
@@ -2076,7 +2076,7 @@ struct AsmFluidArgs {
   float *dchi, *ddchi;       // [n][B]
   // symplectic: the drift of the next stage (or the final drift) right after
   // the kick, chi = chi + dchi*cd_next, axis-masked when drift_mask is set
-  int drift, drift_mask;
+  int drift_mask;
   double cd_next;
   float *chi;                // [n][B]
   // the next step's predictor (first drift), axis-masked with mask_axis, into
@@ -2136,7 +2136,7 @@ __device__ __forceinline__ void fluid_sum(const float *force, int4 c, const int 
 // component's sum still runs over the copies in ascending slot order from
 // zero.  The point's velocity (and acceleration, displacement) is loaded
 // before the gather for the same reason.
-template <int B>
+template <int B, bool NM>
 __device__ __forceinline__ void asm_solid_point(const AsmSolidArgs &A, int ip) {
   const int g = ip < A.ncontig ? ip : A.pts[ip];
   int4 cp = A.copies[g];
@@ -2167,14 +2167,16 @@ __device__ __forceinline__ void asm_solid_point(const AsmSolidArgs &A, int ip) {
 #pragma unroll
   for (int c = 0; c < 3; c++)
     on[c] = (A.comps & (1 << c)) && !((fl & kFlagAxis) && c >= A.mask0 && c <= A.mask1);
-  float v[3][B], a0[3][B], u[3][B];
+  // (newmark2 only predicts with the displacement: wide groups request it after the gather)
+  constexpr bool kLate = NM && B >= 3;
+  float v[3][B], a0[NM ? 3 : 1][B], u[3][B];
 #pragma unroll
   for (int c = 0; c < 3; c++) {
     if (!(A.comps & (1 << c))) continue;
     const size_t p = ((size_t)c * A.n + g) * B;
     ldv<B>(A.velo + p, v[c]);
-    if (A.newmark) ldv<B>(A.acc0 + p, a0[c]);
-    if (A.drift || A.gamma || A.disp_next) ldv<B>(A.disp + p, u[c]);
+    if (NM) ldv<B>(A.acc0 + p, a0[NM ? c : 0]);
+    if (!kLate && (!NM || A.gamma || A.disp_next)) ldv<B>(A.disp + p, u[c]);
   }
   // absorbing boundaries: a -= 2 gamma v + gamma^2 u after the inverse mass
   // (SOLVER/time_evol_wave.F90:468-491,690-711), with v and u of this stage
@@ -2256,8 +2258,12 @@ __device__ __forceinline__ void asm_solid_point(const AsmSolidArgs &A, int ip) {
         for (int b = 0; b < B; b++) s[c][b] = s[c][b] + x[c][b];
   }
   if (fl & kFlagSource) {
-#pragma unroll
-    for (int b = 0; b < B; b++) {
+    // (a loop of hidden length: unrolled or straight, the arguments of all wavefields are
+    // loaded at the kernel's start and held in scalar registers, which then spill)
+    int nb = B;
+    asm volatile("" : "+s"(nb));
+#pragma unroll 1
+    for (int b = 0; b < nb; b++) {
       const float stf = stf_at(A.stf[b], A.step, b, A.nstages, A.stage);
       if (stf == 0.0f || !A.src_tab[b]) continue;
       const int4 e = A.src_tab[b][((unsigned)g * A.src_mul[b]) >> A.src_shift[b]];
@@ -2265,15 +2271,18 @@ __device__ __forceinline__ void asm_solid_point(const AsmSolidArgs &A, int ip) {
       const float val[3] = {__int_as_float(e.y), __int_as_float(e.z), __int_as_float(e.w)};
 #pragma unroll
       for (int c = 0; c < 3; c++)
-        if (A.comps & (1 << c)) s[c][b] = s[c][b] - val[c] * stf;
+#pragma unroll
+        for (int w = 0; w < B; w++)
+          if (w == b && (A.comps & (1 << c))) s[c][w] = s[c][w] - val[c] * stf;
     }
   }
 #pragma unroll
   for (int c = 0; c < 3; c++) {
     if (!(A.comps & (1 << c))) continue;
     const size_t p = ((size_t)c * A.n + g) * B;
+    if (kLate && (A.gamma || A.disp_next)) ldv<B>(A.disp + p, u[c]);
     float a[B];
-    if (A.newmark) {
+    if (NM) {
 #pragma unroll
       for (int b = 0; b < B; b++) {
         if (c == 2 && A.src == AXH_DIPOLE)
@@ -2281,7 +2290,7 @@ __device__ __forceinline__ void asm_solid_point(const AsmSolidArgs &A, int ip) {
         else
           a[b] = -mi * s[c][b];
         if (A.gamma) a[b] = (a[b] - (2.0f * gm) * v[c][b]) - (gm * gm) * u[c][b];
-        v[c][b] = (float)((double)v[c][b] + A.hdt * (double)(a0[c][b] + a[b]));
+        v[c][b] = (float)((double)v[c][b] + A.hdt * (double)(a0[NM ? c : 0][b] + a[b]));
       }
       stv<B>(A.acc0 + p, a);
     } else {
@@ -2296,7 +2305,7 @@ __device__ __forceinline__ void asm_solid_point(const AsmSolidArgs &A, int ip) {
       }
     }
     stv<B>(A.velo + p, v[c]);
-    if (A.drift) {
+    if (!NM) {
       // as k_predict's drift, with the velocity just computed
 #pragma unroll
       for (int b = 0; b < B; b++)
@@ -2320,9 +2329,9 @@ __device__ __forceinline__ void asm_solid_point(const AsmSolidArgs &A, int ip) {
       }
 #pragma unroll
       for (int b = 0; b < B; b++)
-        u[c][b] = A.newmark ? (float)((double)u[c][b] + A.dt * (double)v[c][b] +
-                                      A.hdt2 * (double)a[b])
-                            : (float)((double)u[c][b] + (double)v[c][b] * A.cd0);
+        u[c][b] = NM ? (float)((double)u[c][b] + A.dt * (double)v[c][b] +
+                               A.hdt2 * (double)a[b])
+                     : (float)((double)u[c][b] + (double)v[c][b] * A.cd0);
       if (fl & kFlagAxisBdry) {
         for (int k = 0; k < A.naxb; k++)
           if (A.axb_g[k] == g) stv<B>(A.axb_val + ((size_t)k * 3 + c) * B, u[c]);
@@ -2336,7 +2345,7 @@ __device__ __forceinline__ void asm_solid_point(const AsmSolidArgs &A, int ip) {
   }
 }
 
-template <int B>
+template <int B, bool NM>
 __device__ __forceinline__ void asm_fluid_point(const AsmFluidArgs &A, int g) {
   float s[B];
   const int4 cp = A.copies[g];
@@ -2344,7 +2353,7 @@ __device__ __forceinline__ void asm_fluid_point(const AsmFluidArgs &A, int g) {
   const float mi = A.minv[g];
   float d[B], dd[B], c[B];
   ldv<B>(A.dchi + (size_t)g * B, d);
-  if (A.drift || A.gamma || A.chi_next) ldv<B>(A.chi + (size_t)g * B, c);
+  if (!NM || A.gamma || A.chi_next) ldv<B>(A.chi + (size_t)g * B, c);
   // absorbing boundaries: ddchi -= 2 gamma dchi + gamma^2 chi after the
   // inverse mass (SOLVER/time_evol_wave.F90:432-434,663-665)
   const float gm = A.gamma ? A.gamma[g] : 0.0f;
@@ -2353,7 +2362,7 @@ __device__ __forceinline__ void asm_fluid_point(const AsmFluidArgs &A, int g) {
     dd[b] = -mi * s[b];
     if (A.gamma) dd[b] = (dd[b] - (2.0f * gm) * d[b]) - (gm * gm) * c[b];
   }
-  if (A.newmark) {
+  if (NM) {
     float d0[B];
     ldv<B>(A.ddchi + (size_t)g * B, d0);
 #pragma unroll
@@ -2365,7 +2374,7 @@ __device__ __forceinline__ void asm_fluid_point(const AsmFluidArgs &A, int g) {
   }
   stv<B>(A.ddchi + (size_t)g * B, dd);
   stv<B>(A.dchi + (size_t)g * B, d);
-  if (A.drift) {
+  if (!NM) {
 #pragma unroll
     for (int b = 0; b < B; b++) c[b] = (float)((double)c[b] + (double)d[b] * A.cd_next);
     if (A.drift_mask && (A.flags[g] & kFlagAxis)) {
@@ -2378,8 +2387,8 @@ __device__ __forceinline__ void asm_fluid_point(const AsmFluidArgs &A, int g) {
     const bool masked = A.mask_axis && (A.flags[g] & kFlagAxis);
 #pragma unroll
     for (int b = 0; b < B; b++) {
-      c[b] = A.newmark ? (float)((double)c[b] + A.dt * (double)d[b] + A.hdt2 * (double)dd[b])
-                       : (float)((double)c[b] + (double)d[b] * A.cd0);
+      c[b] = NM ? (float)((double)c[b] + A.dt * (double)d[b] + A.hdt2 * (double)dd[b])
+                : (float)((double)c[b] + (double)d[b] * A.cd0);
       if (masked) c[b] = 0.0f;
     }
     stv<B>(A.chi_next + (size_t)g * B, c);
@@ -2498,34 +2507,42 @@ __global__ __launch_bounds__(256) void k_kwf(KwfArgs A) {
 // newmark2, whose displacement of the step it does not write, takes the
 // step's receiver samples (nrec workgroups per wavefield) and kernel
 // wavefields (nkwf per wavefield).
+//
+// Newmark2 and the symplectic stages are instances of their own (NM): with both in one
+// the widths 3 and 4 spilled 27 and 12 VGPRs to scratch memory and every width 33 to 57
+// SGPRs, 7 workgroups per CU for one wavefield; now none spills and 8 fit.  50 s mesh, 40
+// newmark2 steps 481 -> 463 us; 10 s mesh, 8 symplec4 steps 2773 -> 2708; 4 wavefields, 4 steps
+// 1939 -> 1910.
 // workgroups of k_asm: solid points, fluid points, receivers and kernel
 // wavefields (the last two per wavefield)
 struct AsmBlocks {
   int solid, fluid, rec, kwf;
 };
 
-template <int B>
+template <int B, bool NM>
 __global__ __launch_bounds__(256, (B >= 3 ? 5 : 6))
 void k_asm(AsmSolidArgs A, AsmFluidArgs F, RecArgs R, KwfArgs K, AsmBlocks N) {
   int blk = blockIdx.x;
   if (blk < N.solid) {
     const int ip = xcd_block(blk, N.solid) * 256 + threadIdx.x;
-    if (ip < A.npts) asm_solid_point<B>(A, ip);
+    if (ip < A.npts) asm_solid_point<B, NM>(A, ip);
     return;
   }
   blk -= N.solid;
   if (blk < N.fluid) {
     const int g = xcd_block(blk, N.fluid) * 256 + threadIdx.x;
-    if (g < F.n) asm_fluid_point<B>(F, g);
+    if (g < F.n) asm_fluid_point<B, NM>(F, g);
     return;
   }
-  blk -= N.fluid;
-  if (blk < N.rec * B) {
-    rec_sample<B>(R, (blk / B) * 256 + threadIdx.x, blk % B);
-    return;
+  if constexpr (NM) {
+    blk -= N.fluid;
+    if (blk < N.rec * B) {
+      rec_sample<B>(R, (blk / B) * 256 + threadIdx.x, blk % B);
+      return;
+    }
+    blk -= N.rec * B;
+    kwf_points<B>(K, blk % B, blk / B, N.kwf);
   }
-  blk -= N.rec * B;
-  kwf_points<B>(K, blk % B, blk / B, N.kwf);
 }
 
 // Start of a run that does not begin with k_predict (replayed graphs, initial
@@ -4248,7 +4265,7 @@ static void run_group(Runner &R, const MeshDev &M, Fields &F, Member *const *mb,
   PF.flags = M.flags_f; PF.stride = M.nglob_f; PF.naxb = 0; PF.axb_g = nullptr;
   PF.u = F.chi; PF.v = F.dchi; PF.a0 = F.ddchi; PF.axb_val = F.axb_val;
   AsmSolidArgs AS{};
-  AS.n = M.nglob_s; AS.src = M.src; AS.newmark = newmark; AS.nslot = (int)nslot_s;
+  AS.n = M.nglob_s; AS.src = M.src; AS.nslot = (int)nslot_s;
   AS.comps = comps; AS.mask0 = mask0; AS.mask1 = mask1; AS.gstart = M.gstart_s;
   AS.npts = F.nasm; AS.pts = F.asm_pts;
   // one wavefield: the assembled points are first the mesh's range
@@ -4263,7 +4280,7 @@ static void run_group(Runner &R, const MeshDev &M, Fields &F, Member *const *mb,
   AS.cpl_gf = M.cpl_gf;
   AS.ddchi = M.split_asm ? F.ddchi : nullptr;
   AsmFluidArgs AF{};
-  AF.n = M.nglob_f; AF.newmark = newmark; AF.mask_axis = multipole;
+  AF.n = M.nglob_f; AF.mask_axis = multipole;
   AF.copies = M.copies_f; AF.gstart = M.gstart_f; AF.gslot = M.gslot_f;
   AF.flags = M.flags_f; AF.minv = M.minv_f; AF.hdt = hdt; AF.force = F.force_f;
   AF.gamma = M.gamma_f;
@@ -4346,6 +4363,7 @@ static void run_group(Runner &R, const MeshDev &M, Fields &F, Member *const *mb,
   // segment's last step ends in disp, chi.  With sample_all the receiver
   // samples are taken every step (a graph's steps are all alike), else only
   // where a wavefield takes one (step: the run's step on the host)
+  const auto k_asm_of = newmark ? k_asm<B, true> : k_asm<B, false>;
   float *const dbuf[2] = {F.disp, F.disp2}, *const cbuf[2] = {F.chi, F.chi2};
   auto one_step = [&](int k, int n, bool sample_all, int step) {
     PS.step.koff = PF.step.koff = FA.step.koff = AS.step.koff = RA.step.koff = k;
@@ -4383,7 +4401,6 @@ static void run_group(Runner &R, const MeshDev &M, Fields &F, Member *const *mb,
       // the drifts after the first are fused into the kicks: coefd(st+1),
       // masked except the final one (SOLVER/time_evol_wave.F90:597-605,720-725)
       const bool last = st + 1 == M.nstages;
-      AS.drift = AF.drift = !newmark;
       AS.cd_next = AF.cd_next = newmark ? 0.0 : M.coefd[st + 1];
       AS.drift_mask = !last;
       AF.drift_mask = !last && multipole;
@@ -4400,7 +4417,7 @@ static void run_group(Runner &R, const MeshDev &M, Fields &F, Member *const *mb,
       if (M.split_asm) {
         const AsmBlocks NF{0, N.fluid, 0, 0};
         L(KC_ASM_F, [&] {
-          hipLaunchKernelGGL(k_asm<B>, dim3(NF.fluid), dim3(256), 0, st_, AS, AF, RA, KA, NF);
+          hipLaunchKernelGGL(k_asm_of, dim3(NF.fluid), dim3(256), 0, st_, AS, AF, RA, KA, NF);
         });
         N.fluid = 0;
       }
@@ -4409,7 +4426,7 @@ static void run_group(Runner &R, const MeshDev &M, Fields &F, Member *const *mb,
         N.kwf = snap ? kwf_blocks : 0;
       }
       L(KC_ASM_S, [&] {
-        hipLaunchKernelGGL(k_asm<B>, dim3(N.solid + N.fluid + (N.rec + N.kwf) * B), dim3(256), 0,
+        hipLaunchKernelGGL(k_asm_of, dim3(N.solid + N.fluid + (N.rec + N.kwf) * B), dim3(256), 0,
                            st_, AS, AF, RA, KA, N);
       });
     }
