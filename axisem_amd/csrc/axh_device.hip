@@ -1468,7 +1468,7 @@ void k_solid(SolidArgs A, FluidArgs FA) {
   if (valid) {
     if (direct) {
       // the point's only copy: assembly (0 + f, as the gather sums), kick
-      // and drift as in k_asm_solid
+      // and drift as in asm_solid_point
       const float mi = dmi;
 #pragma unroll
       for (int cc = 0; cc < NCOMP; cc++) {
@@ -4574,9 +4574,9 @@ void device_run(axh_ctx *ctx, int32_t it0, int32_t it1, float *seis) {
 // ---------------------------------------------------------------------------
 constexpr size_t kKwfRingBytes = AXH_KWF_RING_BYTES;  // snapshot ring on the device
 // One pinned staging half: small enough that short runs and small grids move their
-// first snapshots while later steps run (20 s mesh, 26 steps with 3 snapshots of 3
-// MB: halves of 16 MiB 1179, of 4 MiB 1124, of 2 MiB 1150 us; 260 steps with 21
-// 10.1, 9.5, 9.6 ms; 50 s mesh, 30 of 0.8 MB in 60 steps 2239, 1732, 1785 us).
+// first snapshots while later steps run.  Halves of 16 and of 4 MiB: 20 s mesh, 26 steps with 3
+// snapshots of 3 MB 1179, 1124 us; 260 steps with 21 10.1, 9.5 ms; 50 s mesh, 30 of 0.8 MB
+// in 60 steps 2239, 1732 us, and 1785 with 2 MiB (3 MB snapshots are one per half in both).
 constexpr size_t kKwfStageBytes = (size_t)4 << 20;
 
 // The point tables of k_kwf from the context's grid, in point order: the
